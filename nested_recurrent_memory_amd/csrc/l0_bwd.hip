@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void l0_bwd_intra_kernel(L0BwdIntraArgs a) 
   // test-only path) reads them from global memory
   constexpr bool STAGE = !std::is_same<E, float>::value;
   typedef typename Mma<E>::SFrag SF;
-  typedef Mma<float> MF;
+  typedef Mma1 MF;
   // Phases 2-3 hold dX_w, dX_u; phases 4-6 reuse the space for dA, dAqk and,
   // per pass, gc (later its gradient, in place) and the k, b, q columns.
   constexpr size_t SZ_X = sizeof(float) * C * (LXK + LXV);

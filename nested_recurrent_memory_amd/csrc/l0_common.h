@@ -365,7 +365,7 @@ __device__ __forceinline__ void l0_build_A(float* s_A, const float* s_gc,
 // has row stride LDT. Ends with a barrier.
 template <int LDT>
 __device__ __forceinline__ void l0_invert(float* s_A, float* s_T) {
-  typedef Mma<float> MF;
+  typedef Mma1 MF;
   const int lane = lane_id(), wv = wave_id(), tid = threadIdx.x;
   if (wv == 0) {
     const int I = lane >> 4, c = lane & 15, o = 16 * I;

@@ -2,7 +2,7 @@
 //
 // Matrix work runs on the CDNA4 matrix cores through two 16x16 MFMA shapes:
 //   bf16 operands: v_mfma_f32_16x16x32_bf16  (8 k-values per lane)
-//   fp32 operands: v_mfma_f32_16x16x4_f32    (1 k-value per lane)
+//   fp32 operands: v_mfma_f32_16x16x4_f32    (1 k-value per lane; fragments of four)
 // both accumulating in fp32. For a wave (64 lanes) and lane l:
 //   A fragment: row (l & 15), k-values starting at kofs(l) = KPL * (l >> 4)
 //   B fragment: col (l & 15), the same k-values
@@ -127,22 +127,47 @@ template <> struct Mma<bf16> {
   __device__ __forceinline__ static bf16 lo_of(float x, bf16 hi) { return (bf16)(x - (float)hi); }
 };
 
+// fp32: one fragment is 16 k-values, four per lane (lane group g = l / 16
+// holds k = 4 g .. + 3), multiplied by four v_mfma_f32_16x16x4_f32; the e-th
+// takes every lane's e-th value, so its four k-values are e, 4 + e, 8 + e,
+// 12 + e. The order of a sum over k does not matter to the operands as long
+// as A and B agree on it, and so an operand is one 16-byte load (from HBM or
+// LDS) per 16 k-values instead of four 4-byte ones that touch four times the
+// cache lines: one k-value per lane left every fp32 kernel waiting for its
+// operands (forward and backward of the op at B = 2, T = 2048, H = 8,
+// K = 128, two levels: 1582 -> 1014 us a step).
 template <> struct Mma<float> {
+  static constexpr int KS = 16;
+  static constexpr int KPL = 4;
+  typedef f4 Frag;
+  typedef f4 SFrag;
+  __device__ __forceinline__ static f4 mma(f4 acc, f4 a, f4 b) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+    return acc;
+  }
+  __device__ __forceinline__ static f4 ld(const float* p) { return *reinterpret_cast<const f4*>(p); }
+  __device__ __forceinline__ static float elem(const f4& f, int e) { return f[e]; }
+  template <typename F>
+  __device__ __forceinline__ static f4 make(F f) {
+    f4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = f(e);
+    return r;
+  }
+  template <typename F>
+  __device__ __forceinline__ static f4 makes(F f) { return make(f); }
+  __device__ __forceinline__ static f4 zero() { return f4_zero(); }
+  __device__ __forceinline__ static f4 szero() { return f4_zero(); }
+};
+
+// One fp32 MFMA on scalar fragments (k-value l / 16 of a lane), for operands
+// formed one value at a time: the decay backward and the block inversion.
+struct Mma1 {
   static constexpr int KS = 4;
-  static constexpr int KPL = 1;
-  typedef float Frag;
-  typedef float SFrag;
   __device__ __forceinline__ static f4 mma(f4 acc, float a, float b) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
   }
-  __device__ __forceinline__ static float ld(const float* p) { return *p; }
-  __device__ __forceinline__ static float elem(float f, int) { return f; }
-  template <typename F>
-  __device__ __forceinline__ static float make(F f) { return f(0); }
-  template <typename F>
-  __device__ __forceinline__ static float makes(F f) { return f(0); }
-  __device__ __forceinline__ static float zero() { return 0.f; }
-  __device__ __forceinline__ static float szero() { return 0.f; }
 };
 
 // An LDS tile of derived (fp32) values kept in the form the matrix core
@@ -185,7 +210,7 @@ template <> struct SplitTile<float> {
     *reinterpret_cast<f4*>(p + off) = x;
   }
   __device__ __forceinline__ void put1(int off, float x) const { p[off] = x; }
-  __device__ __forceinline__ float get(int off) const { return p[off]; }
+  __device__ __forceinline__ f4 get(int off) const { return *reinterpret_cast<const f4*>(p + off); }
 };
 
 // Derived operands that only ever enter the matrix core are also kept in HBM
@@ -240,11 +265,13 @@ __device__ __forceinline__ f4 mma_tile(f4 acc, const TA* A, int lda, const TB* B
   return acc;
 }
 
-// Mma<E>::KPL consecutive elements at p as floats (one 16-byte load for bf16).
+// Mma<E>::KPL consecutive elements at p as floats (one 16-byte load).
 template <typename E>
 __device__ __forceinline__ void ld_vals(const E* p, float* out) {
   if constexpr (std::is_same<E, float>::value) {
-    out[0] = *p;
+    const f4 v = *reinterpret_cast<const f4*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = v[e];
   } else {
     const bf16x8 v = *reinterpret_cast<const bf16x8*>(p);
 #pragma unroll
@@ -346,14 +373,10 @@ __device__ __forceinline__ void head_xcd_split(int x, int H, int NF, int& b, int
 // a row-major array staged in LDS. Exact (E) or derived (fp32) storage.
 template <typename E>
 __device__ __forceinline__ typename Mma<E>::Frag gather_x(const E* p, int ld) {
-  if constexpr (std::is_same<E, float>::value) {
-    return p[0];
-  } else {
-    typename Mma<E>::Frag r;
+  typename Mma<E>::Frag r;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = p[e * ld];
-    return r;
-  }
+  for (int e = 0; e < Mma<E>::KPL; ++e) r[e] = p[e * ld];
+  return r;
 }
 template <typename E>
 __device__ __forceinline__ typename Mma<E>::SFrag gather_s(const float* p, int ld) {

@@ -146,13 +146,7 @@ __global__ __launch_bounds__(512) void promote_chain_kernel(PromoteChainArgs a) 
 #pragma unroll
       for (int s = 0; s < NKS; ++s) {
         const float* p = Sh + (unsigned)(v * K + s * KS + kofs<E>(ln));
-        if constexpr (KPL == 8) {
-          const f4 x0 = *reinterpret_cast<const f4*>(p), x1 = *reinterpret_cast<const f4*>(p + 4);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) { raw[s * KPL + e] = x0[e]; raw[s * KPL + 4 + e] = x1[e]; }
-        } else {
-          raw[s * KPL] = *p;
-        }
+        ld_raw<KPL>(p, raw + s * KPL);
       }
     }
   };

@@ -448,10 +448,10 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
   typedef E DV __attribute__((__vector_size__(DOE * sizeof(E))));
   constexpr int FK = BF ? 1 : NSK, FM = BF ? 1 : NSM, FT = BF ? 1 : TRT;
   struct Ops {
-    float kt[FK];               // fp32: Kt rows of this wave's dVn tile, transposed reads
-    float aq[FM];               // fp32: Aqk^T rows
-    float wt[FT][FM];           // fp32: W^T rows of this wave's state tiles
-    float qg[FT][FM];           // fp32: Qg^T rows
+    f4 kt[FK];                  // fp32: Kt rows of this wave's dVn tile, transposed reads
+    f4 aq[FM];                  // fp32: Aqk^T rows
+    f4 wt[FT][FM];              // fp32: W^T rows of this wave's state tiles
+    f4 qg[FT][FM];              // fp32: Qg^T rows
     float g[TRT][4];
     DV dor;                     // do at this thread's staging slots, raw
     E dm;                       // and mix_0 of its token, raw (converted when staged)
@@ -470,23 +470,27 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
       CW::template load<K>(wq, NCW * wv, pre + 2 * (CK::NL + CQ::NL));
       CW::template load<K>(qq, NCW * wv, pre + 2 * (CK::NL + CQ::NL + CW::NL));
     } else {
-      // element (row tile rt of X^T, k = 4 s + lane / 16) = X[4 s + lane / 16][16 rt + lane % 16]
+      // element e of a fragment (row tile rt of X^T, k = 16 s + 4 (lane / 16) + e)
+      // = X[k][16 rt + lane % 16]
       const float* kt = tile(a.KtT, j, K * M);
       const float* aq = tile(a.Aqk, j, M * M);
       const float* wq = tile(a.W, j, M * K);
       const float* qq = tile(a.Qg, j, M * K);
-      const int lr = lane >> 4, lc = lane & 15;
+      const int lr = 4 * (lane >> 4), lc = lane & 15;
 #pragma unroll
-      for (int s = 0; s < FK; ++s) o.kt[s] = kt[(4 * s + lr) * M + 16 * wv + lc];
+      for (int e = 0; e < 4; ++e) {
 #pragma unroll
-      for (int s = 0; s < FM; ++s) o.aq[s] = aq[(4 * s + lr) * M + 16 * wv + lc];
+        for (int s = 0; s < FK; ++s) o.kt[s][e] = kt[(16 * s + lr + e) * M + 16 * wv + lc];
 #pragma unroll
-      for (int t = 0; t < FT; ++t)
+        for (int s = 0; s < FM; ++s) o.aq[s][e] = aq[(16 * s + lr + e) * M + 16 * wv + lc];
 #pragma unroll
-        for (int s = 0; s < FM; ++s) {
-          o.wt[t][s] = wq[(4 * s + lr) * K + NCW * wv + 16 * t + lc];
-          o.qg[t][s] = qq[(4 * s + lr) * K + NCW * wv + 16 * t + lc];
-        }
+        for (int t = 0; t < FT; ++t)
+#pragma unroll
+          for (int s = 0; s < FM; ++s) {
+            o.wt[t][s][e] = wq[(16 * s + lr + e) * K + NCW * wv + 16 * t + lc];
+            o.qg[t][s][e] = qq[(16 * s + lr + e) * K + NCW * wv + 16 * t + lc];
+          }
+      }
     }
     const float* Gj = Gb + (size_t)j * K;
 #pragma unroll
