@@ -332,6 +332,12 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Waits for every global access issued so far (the compiler counts from
+// there). Ahead of a loop whose first step's operands are loaded before it:
+// the loop's waits are then counted from its own order of loads and stores
+// rather than from the shorter one at its entry.
+__device__ __forceinline__ void wait_global() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0)
+
 // Splits a grid of G = NB * NS blocks into (b, s), b in [0, NB), s in [0, NS),
 // so that the NS slices of one b run on the same XCD (blocks are dealt to the
 // 8 XCDs round robin, block x on XCD x % 8). Falls back to b = x / NS when
@@ -440,6 +446,26 @@ __device__ __forceinline__ void stage_split(const ST& dst, int ld, const float* 
     const int e = threadIdx.x + NTH * u, r = e / SEGS, c = (e % SEGS) * 4;
     if (NSEG % NTH == 0 || e < NSEG) dst.put4(r * ld + c, x[u]);
   }
+}
+
+// ---------------------------------------------------------------- buffer access
+//
+// Global accesses through a buffer descriptor: an access past the
+// descriptor's bytes is dropped (a load gives 0) instead of being branched
+// around, so that the instruction is always issued. The scans need that:
+// loads and stores share one in-order counter (vmcnt), and with a store under
+// a branch the compiler cannot know how many of them follow the next step's
+// operand loads, so it waits for every store of the step as well. The base
+// must be uniform over the wave; offsets are bytes from it, below 2^31.
+typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u4;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf(const void* base, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int ofs, float x) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, ofs, 0, 0);
+}
+__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int ofs, f4 x) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, ofs, 0, 0);
 }
 
 // ---------------------------------------------------------------- misc

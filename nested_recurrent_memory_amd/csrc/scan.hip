@@ -20,13 +20,6 @@
 // product is three bf16 MFMAs on split operands.
 #include "ngdn_kernels.h"
 
-#ifndef SCAN_WAVES_128
-#define SCAN_WAVES_128 4
-#endif
-#ifndef SCAN_LATE_STORES
-#define SCAN_LATE_STORES 1
-#endif
-
 namespace ngdn {
 
 // OUT (level 0): each step also forms the chunk's level-0 read
@@ -36,7 +29,16 @@ namespace ngdn {
 // sequence nor Vn from HBM).
 // FRM (bf16): bit 0, BT in fragment order (M % 32 == 0); bit 1, A (and, OUT,
 // Qg and Aqk) too.
-template <typename E, int K, int M, int BV, int NWV, bool OUT, int FRM>
+// SM, the outputs of a step: 1, level 0 without a backward (read0, and the
+// transposed state where it is due); 2, level 0 with one (also the state and
+// Vn); 3, an upper level (the state, and its transpose when set). These issue
+// every store of a step unconditionally (buffer stores, dropped where not
+// due) and run two steps per loop iteration on two operand sets, so that a
+// step waits for its own operands only: with stores under branches and one
+// set copied to the next at the loop's end, every step waited for all of its
+// own stores as well. 0, any set of outputs, each store under its condition
+// (the entry points' less common calls).
+template <typename E, int K, int M, int BV, int NWV, bool OUT, int FRM, int SM>
 __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
   constexpr int CT = BV / 16;                 // column tiles
   constexpr int RTS = K / 16;                 // state row tiles
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
       const int g = wv + NWV * p;
       rt = g % RTV;
       ct = g / RTV;
-      return g < NVT;
+      return NVT % NWV == 0 || g < NVT;   // (a test the compiler cannot resolve would branch)
     }
     rt = wv + NWV * (p / CT);
     ct = p % CT;
@@ -159,9 +161,33 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
     }
   };
 
+  // SM: the next step whose transposed state is due
+  const int vk_step = a.vk_every > 1 ? a.vk_every : 1;
+  int vk_next = SM ? (a.j0 + vk_step - 1) / vk_step * vk_step : 0;
   auto store_state = [&](int j) {
-    const size_t base = (a.state_mode == 0 ? (size_t)bh * S + j
-                                           : ((size_t)b * a.NG + j) * H + h) * K * V;
+    // (SM: the mode is known, so no branch stands between a product and the
+    // stores of its result: across one, this compiler left out the wait
+    // states that an MFMA's result needs before it is read)
+    const bool by_chunk = SM == 0 ? a.state_mode == 0 : SM < 3;
+    const size_t base = (by_chunk ? (size_t)bh * S + j
+                                  : ((size_t)b * a.NG + j) * H + h) * K * V;
+    if constexpr (SM != 0) {
+      const bool due = a.st_vk && j == vk_next;
+      if (j == vk_next) vk_next += vk_step;
+      const auto rvk = buf(a.st_vk + base, due ? K * V * 4 : 0);
+      const auto rkv = buf(a.st_kv + base, K * V * 4);
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        const int g = wv * TPW + i, rt = g / CT, ct = g % CT;
+        const int k0 = rt * 16 + acc_row(0), v = v0 + ct * 16 + acc_col();
+        buf_st(rvk, (v * K + k0) * 4, st[i]);
+        if constexpr (SM >= 2) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) buf_st(rkv, ((k0 + r) * V + v) * 4, st[i][r]);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int g = wv * TPW + i, rt = g / CT, ct = g % CT;
@@ -175,39 +201,51 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
     }
   };
 
-  // Vn and (OUT) the read of a step are stored at the start of the next
-  // step, beside the state entering it and ahead of that step's operand
-  // loads: the vector memory pipe is in order, so stores issued after the
-  // loads would wait for them to drain and hold the wave up mid-step.
-  // (fp32 operands with K = 128 and M >= 64 keep the stores in place: the
-  // held Vn tiles would not fit in their registers)
-  constexpr bool DEFER = OUT || sizeof(E) == 2 || K < 128 || M < 64;
-  // LATE: stores after the step's products instead of at its start
-  constexpr bool LATE = SCAN_LATE_STORES && DEFER;
+  // A step's stores follow its products, while the next step's operand loads
+  // (issued before them) are in flight: the vector memory pipe is in order,
+  // so stores ahead of the loads would hold those up, and stores between the
+  // products would hold the wave.
   f4 pvn[NVP], prd[OUT ? NVP : 1];
-  auto flush_tile = [&](int jj, int p) {
-      int rt, ct;
-      if (vn_tile(p, rt, ct)) {
-        const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-        if (a.vnT)
-          *reinterpret_cast<f4*>(a.vnT + (((size_t)bh * S + jj) * V + v0 + vl) * M + m0) = pvn[p];
-        if (a.vn) {
-          float* vp = a.vn + ((size_t)bh * S + jj) * M * V + (size_t)m0 * V + v0 + vl;
+  auto flush = [&](int jj) {
+    if constexpr (SM != 0) {
+      const auto rvn = buf(a.vn + ((size_t)bh * S + jj) * M * V, M * V * 4);
+      // rows of the chunk inside the sequence
+      const int rows = min(M, a.T - jj * M);
+      const auto rrd = buf(a.read0 + (((size_t)b * a.T + (size_t)jj * M) * H + h) * V,
+                           (unsigned)(((rows - 1) * H + 1) * V * 4));
 #pragma unroll
-          for (int r = 0; r < 4; ++r) vp[(size_t)r * V] = pvn[p][r];
-        }
-        if constexpr (OUT) {
+      for (int p = 0; p < NVP; ++p) {
+        int rt, ct;
+        if (!vn_tile(p, rt, ct)) continue;
+        const int m0 = rt * 16 + acc_row(0), v = v0 + ct * 16 + acc_col();
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int t = jj * M + rt * 16 + acc_row(r);
-            if (t < a.T) a.read0[(((size_t)b * a.T + t) * H + h) * V + v0 + vl] = prd[p][r];
-          }
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (SM == 2) buf_st(rvn, ((m0 + r) * V + v) * 4, pvn[p][r]);
+          if constexpr (OUT) buf_st(rrd, ((m0 + r) * H * V + v) * 4, prd[p][r]);
         }
       }
-  };
-  auto flush = [&](int jj) {
+      return;
+    }
 #pragma unroll
-    for (int p = 0; p < NVP; ++p) flush_tile(jj, p);
+    for (int p = 0; p < NVP; ++p) {
+      int rt, ct;
+      if (!vn_tile(p, rt, ct)) continue;
+      const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
+      if (a.vnT)
+        *reinterpret_cast<f4*>(a.vnT + (((size_t)bh * S + jj) * V + v0 + vl) * M + m0) = pvn[p];
+      if (a.vn) {
+        float* vp = a.vn + ((size_t)bh * S + jj) * M * V + (size_t)m0 * V + v0 + vl;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vp[(size_t)r * V] = pvn[p][r];
+      }
+      if constexpr (OUT) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = jj * M + rt * 16 + acc_row(r);
+          if (t < a.T) a.read0[(((size_t)b * a.T + t) * H + h) * V + v0 + vl] = prd[p][r];
+        }
+      }
+    }
   };
 
   // One step with its operands already loaded.
@@ -244,7 +282,6 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
           for (int r = 0; r < 4; ++r) vn[r] = cur.u[p][r] - acc[r];
           sVn.put4(vl * LDS_VN + m0, vn);
           pvn[p] = vn;
-          if constexpr (!DEFER) flush_tile(j, p);
         }
       }
       lds_barrier();
@@ -264,14 +301,10 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
           }
         }
       }
-      if constexpr (LATE) {
-        // ---- this step's stores after its products, while the next step's
-        // operand loads (issued before them) are in flight: the stores neither
-        // hold the wave up behind those loads nor delay their completion. The
-        // state registers still hold the state entering step j.
-        store_state(j);
-        flush(j);
-      }
+      // ---- this step's stores (the state registers still hold the state
+      // entering step j)
+      store_state(j);
+      flush(j);
 
       // ---- S <- diag(gam) S + BT Vn
 #pragma unroll
@@ -296,27 +329,33 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
     // the next writes to s_vn follow the next step's barrier
   };
 
-  Ops nxt;
-  // steps [j0, j1): the state registers start from init, the state entering j0
+  // steps [j0, j1): the state registers start from init, the state entering
+  // j0. Each step's operand loads are issued a step ahead, unconditionally (the
+  // last step reloads its own, so that no branch guards them).
   const int j0 = a.j0, j1 = a.j1 > 0 ? a.j1 : S;
-  if (j1 > j0) load(j0, nxt);
-  for (int j = j0; j < j1; ++j) {
-    const Ops cur = nxt;
-    if constexpr (LATE) {
-      // ---- the next step's operand loads first (the last step reloads its
-      // own, so that no branch guards them); this step's stores follow its
-      // products
-      load(j + 1 < j1 ? j + 1 : j, nxt);
-    } else {
-      // ---- state entering step j (and the previous step's Vn and read) to
-      // global, then the next step's operand loads
-      store_state(j);
-      if (DEFER && j > j0) flush(j - 1);
-      if (j + 1 < j1) load(j + 1, nxt);
+  if constexpr (SM != 0) {
+    Ops x, y;
+    if (j1 > j0) load(j0, x);
+    wait_global();
+    int j = j0;
+    for (; j + 1 < j1; j += 2) {
+      load(j + 1, y);
+      __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step
+      step(j, x);
+      load(j + 2 < j1 ? j + 2 : j + 1, x);
+      __builtin_amdgcn_sched_barrier(0);
+      step(j + 1, y);
     }
-    step(j, cur);
+    if (j < j1) step(j, x);
+  } else {
+    Ops nxt;
+    if (j1 > j0) load(j0, nxt);
+    for (int j = j0; j < j1; ++j) {
+      const Ops cur = nxt;
+      load(j + 1 < j1 ? j + 1 : j, nxt);
+      step(j, cur);
+    }
   }
-  if (!LATE && DEFER && j1 > j0) flush(j1 - 1);
   if (a.state_mode == 1 && j1 == S) {
     for (int j = S; j < a.NG; ++j) store_state(j);
   }
@@ -334,60 +373,69 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
 
 // Waves per workgroup: four, one per SIMD. Eight (two per SIMD) leave each
 // wave half the registers, less than a step's operands read ahead need.
-template <int K> constexpr int scan_waves() { return K == 128 ? SCAN_WAVES_128 : 4; }
+constexpr int SCAN_WAVES = 4;
 
-template <typename E, int K, int M, int BV>
-static hipError_t launch_scan_bv(const ScanArgs& a, hipStream_t st) {
-  constexpr int NWV = scan_waves<K>();
+// The outputs of a call (SM above). The buffer stores of read0 take a chunk's
+// rows as byte offsets below 2^31.
+static int scan_outputs(const ScanArgs& a) {
+  if (a.gate.pos || a.vnT) return 0;
+  if (a.read0) {
+    if (a.state_mode != 0 || (long long)a.H * a.V * CH * 4 >= (1LL << 31)) return 0;
+    return a.st_kv && a.vn ? 2 : !a.st_kv && !a.vn ? 1 : 0;
+  }
+  return a.state_mode == 1 && a.st_kv && !a.vn ? 3 : 0;
+}
+
+template <typename E, int K, int M, int BV, bool OUT, int FRM, int SM>
+static hipError_t launch_scan_sm(const ScanArgs& a, hipStream_t st) {
   const unsigned grid = (unsigned)(a.B * a.H * (a.V / BV));
-  constexpr bool BF = std::is_same<E, bf16>::value;
-  if (a.frag && !(BF && M % 32 == 0 && (a.frag == 1 || (a.frag == 3 && M == CH))))
-    return hipErrorInvalidValue;
+  hipLaunchKernelGGL((scan_fwd_kernel<E, K, M, BV, SCAN_WAVES, OUT, FRM, SM>), dim3(grid),
+                     dim3(SCAN_WAVES * WAVE), 0, st, a);
+  return hipGetLastError();
+}
+
+template <typename E, int K, int M, int BV, int FRM>
+static hipError_t launch_scan_frm(const ScanArgs& a, int sm, hipStream_t st) {
   // level 0's read is formed only by the chunk-step (M == CH) kernels whose
   // operand groups share one layout (frag 0 or 3)
-  if (a.read0 && (M != CH || a.frag == 1)) return hipErrorInvalidValue;
-  if constexpr (BF && M == CH) {
-    if (a.frag == 3) {
-      if (a.read0)
-        hipLaunchKernelGGL((scan_fwd_kernel<E, K, M, BV, NWV, true, 3>), dim3(grid),
-                           dim3(NWV * WAVE), 0, st, a);
-      else
-        hipLaunchKernelGGL((scan_fwd_kernel<E, K, M, BV, NWV, false, 3>), dim3(grid),
-                           dim3(NWV * WAVE), 0, st, a);
-      return hipGetLastError();
+  if constexpr (M == CH && FRM != 1) {
+    if (sm == 1) return launch_scan_sm<E, K, M, BV, true, FRM, 1>(a, st);
+    if (sm == 2) return launch_scan_sm<E, K, M, BV, true, FRM, 2>(a, st);
+    if constexpr (BV == SCAN_BV) {
+      if (a.read0) return launch_scan_sm<E, K, M, BV, true, FRM, 0>(a, st);
     }
+  }
+  if (a.read0) return hipErrorInvalidValue;
+  if constexpr (FRM != 3) {
+    if (sm == 3) return launch_scan_sm<E, K, M, BV, false, FRM, 3>(a, st);
+  }
+  if constexpr (BV == SCAN_BV) return launch_scan_sm<E, K, M, BV, false, FRM, 0>(a, st);
+  return hipErrorInvalidValue;
+}
+
+template <typename E, int K, int M, int BV>
+static hipError_t launch_scan_bv(const ScanArgs& a, int sm, hipStream_t st) {
+  constexpr bool BF = std::is_same<E, bf16>::value;
+  if constexpr (BF && M == CH) {
+    if (a.frag == 3) return launch_scan_frm<E, K, M, BV, 3>(a, sm, st);
   }
   if constexpr (BF && M % 32 == 0) {
-    if (a.frag == 1) {
-      hipLaunchKernelGGL((scan_fwd_kernel<E, K, M, BV, NWV, false, 1>), dim3(grid),
-                         dim3(NWV * WAVE), 0, st, a);
-      return hipGetLastError();
-    }
+    if (a.frag == 1) return launch_scan_frm<E, K, M, BV, 1>(a, sm, st);
   }
-  if constexpr (M == CH) {
-    if (a.read0) {
-      hipLaunchKernelGGL((scan_fwd_kernel<E, K, M, BV, NWV, true, 0>), dim3(grid),
-                         dim3(NWV * WAVE), 0, st, a);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((scan_fwd_kernel<E, K, M, BV, NWV, false, 0>), dim3(grid),
-                     dim3(NWV * WAVE), 0, st, a);
-  return hipGetLastError();
+  if (a.frag) return hipErrorInvalidValue;
+  return launch_scan_frm<E, K, M, BV, 0>(a, sm, st);
 }
 
 template <typename E, int K, int M>
 static hipError_t launch_scan(const ScanArgs& a, hipStream_t st) {
-  // Few (batch, head) pairs (a long sequence in a small batch): the bf16
-  // matrix-core paths take 16-column slices, twice the workgroups with half
-  // the products per step each; a step's operands are then read by twice as
-  // many workgroups, which costs more than it saves once the grid fills the
-  // chip.
-  if constexpr (std::is_same<E, bf16>::value && M % 32 == 0) {
-    if (a.frag && a.B * a.H * (a.V / SCAN_BV) <= SCAN_NARROW_GRID)
-      return launch_scan_bv<E, K, M, 16>(a, st);
-  }
-  return launch_scan_bv<E, K, M, SCAN_BV>(a, st);
+  // Few (batch, head) pairs (a long sequence in a small batch): 16-column
+  // slices, twice the workgroups with half the products per step each; a
+  // step's operands are then read by twice as many workgroups, which costs
+  // more than it saves once the grid fills the chip.
+  const int sm = scan_outputs(a);
+  if (sm && a.B * a.H * (a.V / SCAN_BV) <= SCAN_NARROW_GRID)
+    return launch_scan_bv<E, K, M, 16>(a, sm, st);
+  return launch_scan_bv<E, K, M, SCAN_BV>(a, sm, st);
 }
 
 hipError_t scan_fwd(const ScanArgs& a, int dtype, int K, hipStream_t st) {

@@ -108,24 +108,33 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
   const float* Ab = a.AT + (size_t)bh * S * K * M;
   const float* Gb = a.gam + (size_t)bh * S * K;
 
-  // Operands of one step, read a step ahead: they do not depend on the state gradient.
+  // Operands of one step, read a step ahead: they do not depend on the state
+  // gradient. Two sets, one per step of a loop iteration (as in the forward
+  // scan: copying one set to the other at the loop's end made every step wait
+  // for its own stores). The injection, loaded under a branch, comes first:
+  // what is issued after it is then always the same, and the waits for the
+  // operands are exact.
   typedef typename Mma<E>::SFrag SF;
   struct Ops {
     SF bop[RPW][NSK];           // Bop rows of this wave's dVn tiles
     SF at[TRT][NSM];            // A^T rows of this wave's state tiles
-    float g[TRT][4];
+    f4 g[TRT];
     f4 add[TPW];                // the read gradient of the group the step starts
     f4 inj[TPW];                // and, when has_inj, the injection into it
     bool has_inj;
   };
+  constexpr bool ALLV = RTV % 4 == 0;          // every wave has all its dVn tiles
   auto load = [&](int j, Ops& o) {
     const SplitTile<E> Bj = split_at<E>(Bb + (size_t)j * M * K, M * K);
     const SplitTile<E> Aj = split_at<E>(Ab + (size_t)j * K * M, K * M);
     const float* Gj = Gb + (size_t)j * K;
+    const float* ip = inj_tile(j);
+    o.has_inj = ip != nullptr;
+    if (o.has_inj) read_kv(ip, o.inj);
 #pragma unroll
     for (int p = 0; p < RPW; ++p) {
       const int rt = wv + 4 * p;
-      if (rt < RTV) {
+      if (ALLV || rt < RTV) {
         const int brow = (rt * 16 + (lane & 15)) * K + kofs<E>(lane);
 #pragma unroll
         for (int s = 0; s < NSK; ++s) o.bop[p][s] = Bj.get(brow + s * KS);
@@ -140,61 +149,21 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
         o.at[t][s] = FRB ? Aj.get(frag_at(rt, s, M))
                         : (!PADM || s * KS + kofs<E>(lane) < M) ? Aj.get(arow + s * KS)
                                                                 : Mma<E>::szero();
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o.g[t][r] = Gj[rt * 16 + acc_row(r)];
+      o.g[t] = *reinterpret_cast<const f4*>(Gj + rt * 16 + acc_row(0));
     }
     read_kv(dstates(j), o.add);
-    const float* ip = inj_tile(j);
-    o.has_inj = ip != nullptr;
-    if (o.has_inj) read_kv(ip, o.inj);
   };
 
-  // dVn of a step is stored at the start of the step after it, beside dS',
-  // ahead of that step's operand loads: the vector memory pipe is in order,
-  // so stores issued after the loads would wait for them to drain and hold
-  // the wave up mid-step. (M = K = 128 keeps the stores in place: its
-  // registers are already short.)
-  constexpr bool DEFER = !(K == 128 && M == 128);
-  f4 pdv[RPW][CT];
-  auto store_dv = [&](int jj, int p, int ct) {
-    const int rt = wv + 4 * p;
-    const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-    if (a.dVn) {
-      float* o = a.dVn + ((size_t)bh * S + jj) * M * V + (size_t)m0 * V + v0 + vl;
+  auto step = [&](int j, const Ops& cur) {
+    // the group's read gradient and the injection into it (the branch stands
+    // ahead of the products, not between one and the use of its result)
+    f4 add[TPW];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[(size_t)r * V] = pdv[p][ct][r];
+    for (int i = 0; i < TPW; ++i) add[i] = cur.add[i];
+    if (cur.has_inj) {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) add[i] += cur.inj[i];
     }
-    if (a.dVnT)
-      *reinterpret_cast<f4*>(a.dVnT + (((size_t)bh * S + jj) * V + v0 + vl) * M + m0) = pdv[p][ct];
-  };
-  auto flush_dv = [&](int jj) {
-#pragma unroll
-    for (int p = 0; p < RPW; ++p) {
-      if (wv + 4 * p < RTV) {
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) store_dv(jj, p, ct);
-      }
-    }
-  };
-
-  Ops nxt;
-  if (S > 0) load(S - 1, nxt);
-  for (int j = S - 1; j >= 0; --j) {
-    const Ops cur = nxt;
-
-    // ---- dS' (and the previous step's dVn) to global, then the next step's
-    // operand loads
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int g = wv * TPW + i, rt = g / CT, ct = g % CT;
-      const int k0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-      float* o = a.dSp + ((size_t)bh * S + j) * K * V + (size_t)k0 * V + v0 + vl;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[(size_t)r * V] = ds[i][r];
-    }
-    if (DEFER && j + 1 < S) flush_dv(j + 1);
-    if (j > 0) load(j - 1, nxt);
-
     // ---- dS' staged (transposed) as the B operand of Bop dS'
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
@@ -205,10 +174,11 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
     lds_barrier();
 
     // ---- dVn = Bop dS'
+    f4 dv[RPW][CT];
 #pragma unroll
     for (int p = 0; p < RPW; ++p) {
       const int rt = wv + 4 * p;
-      if (rt < RTV) {
+      if (ALLV || rt < RTV) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
           f4 acc = f4_zero();
@@ -218,12 +188,34 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
             acc = Mma<E>::mma(acc, cur.bop[p][s], sdS.get(srow + s * KS));
           const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
           sdV.put4(vl * LDS_VN + m0, acc);
-          pdv[p][ct] = acc;
-          if constexpr (!DEFER) store_dv(j, p, ct);
+          dv[p][ct] = acc;
         }
       }
     }
     lds_barrier();
+
+    // ---- dS' (the state gradient still holds it) and dVn to global
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      const int g = wv * TPW + i, rt = g / CT, ct = g % CT;
+      const int k0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
+      float* o = a.dSp + ((size_t)bh * S + j) * K * V + (size_t)k0 * V + v0 + vl;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[(size_t)r * V] = ds[i][r];
+    }
+#pragma unroll
+    for (int p = 0; p < RPW; ++p) {
+      const int rt = wv + 4 * p;
+      if (ALLV || rt < RTV) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
+          float* o = a.dVn + ((size_t)bh * S + j) * M * V + (size_t)m0 * V + v0 + vl;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[(size_t)r * V] = dv[p][ct][r];
+        }
+      }
+    }
 
     // ---- dS = diag(gam) dS' - A^T dVn, then the group's read gradient
 #pragma unroll
@@ -238,16 +230,38 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
         if (live) fb = sdV.get(vrow + s * KS);
         acc = Mma<E>::mma(acc, cur.at[t][s], fb);
       }
-      f4 add = cur.add[i];
-      if (cur.has_inj) add += cur.inj[i];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) ds[i][r] = cur.g[t][r] * ds[i][r] - acc[r] + add[r];
+      for (int r = 0; r < 4; ++r) ds[i][r] = cur.g[t][r] * ds[i][r] - acc[r] + add[i][r];
     }
     // no barrier here: the next step's writes of s_dst follow this step's
     // second barrier, after every read of s_dst, and its writes of s_dvn
     // follow the next step's first barrier, after every read of s_dvn
+  };
+
+  if constexpr (K == 128 && M == 128) {
+    // two sets would not fit the registers
+    Ops nxt;
+    if (S > 0) load(S - 1, nxt);
+    for (int j = S - 1; j >= 0; --j) {
+      const Ops cur = nxt;
+      load(j > 0 ? j - 1 : 0, nxt);
+      step(j, cur);
+    }
+  } else {
+    Ops x, y;
+    if (S > 0) load(S - 1, x);
+    wait_global();
+    int j = S - 1;
+    for (; j > 0; j -= 2) {
+      load(j - 1, y);
+      __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step
+      step(j, x);
+      load(j > 1 ? j - 2 : 0, x);
+      __builtin_amdgcn_sched_barrier(0);
+      step(j - 1, y);
+    }
+    if (j == 0) step(0, x);
   }
-  if (DEFER && S > 0) flush_dv(0);
   if (a.dinit) {
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
@@ -373,7 +387,11 @@ struct SliceCopy {
   }
 };
 
-template <typename E, int K, int BV>
+// FUSED: only dVn^T leaves (the one-launch chunk backward); otherwise each of
+// dVn and dVn^T that is set. The step's loads are unconditional but for the
+// injection, which comes first, and (FUSED) so are its stores: the wait for
+// the next step's operands is then for them alone (see scan.hip).
+template <typename E, int K, int BV, bool FUSED>
 __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
   constexpr int M = CH;
   constexpr int CT = BV / 16;
@@ -445,21 +463,28 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
   // the chunk's tile of a [B*H,S,R,C] split tensor
   auto tile = [&](const float* X, int j, int RC) { return X + ((size_t)bh * S + j) * RC; };
 
-  typedef E DV __attribute__((__vector_size__(DOE * sizeof(E))));
+  // raw bits: converted where they are used (16-bit registers would be copied,
+  // and the copy waits for the load)
+  constexpr int DOW = DOE * (int)sizeof(E) / 4;
+  typedef __attribute__((__vector_size__(DOW * 4))) int DV;
+  typedef E DE __attribute__((__vector_size__(DOE * sizeof(E))));
   constexpr int FK = BF ? 1 : NSK, FM = BF ? 1 : NSM, FT = BF ? 1 : TRT;
   struct Ops {
     f4 kt[FK];                  // fp32: Kt rows of this wave's dVn tile, transposed reads
     f4 aq[FM];                  // fp32: Aqk^T rows
     f4 wt[FT][FM];              // fp32: W^T rows of this wave's state tiles
     f4 qg[FT][FM];              // fp32: Qg^T rows
-    float g[TRT][4];
+    f4 g[TRT];
     DV dor;                     // do at this thread's staging slots, raw
-    E dm;                       // and mix_0 of its token, raw (converted when staged)
+    int dm;                     // and mix_0 of its token, raw (converted when staged)
+    bool live;                  // whether that token is in the sequence
     f4 add[TPW];                // injection of the step
     bool has_add;
   };
   R16 pre[BF ? NSEG : 1];       // bf16: the next step's slice segments, raw
   auto load = [&](int j, Ops& o) {
+    o.has_add = a.inj && (j + 1) % a.inj_every == 0 && (j + 1) / a.inj_every <= a.inj_nf;
+    if (o.has_add) read_kv(a.inj + ((size_t)bh * a.inj_nf + (j + 1) / a.inj_every - 1) * K * V, o.add);
     if constexpr (BF) {
       const bf16* kt = reinterpret_cast<const bf16*>(tile(a.KtT, j, K * M));
       const bf16* aq = reinterpret_cast<const bf16*>(tile(a.Aqk, j, M * M));
@@ -494,22 +519,16 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
     }
     const float* Gj = Gb + (size_t)j * K;
 #pragma unroll
-    for (int t = 0; t < TRT; ++t) {
-      const int rt = wv * TRT + t;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o.g[t][r] = Gj[rt * 16 + acc_row(r)];
-    }
-    // DOE consecutive columns of one token per thread: one vector load
+    for (int t = 0; t < TRT; ++t)
+      o.g[t] = *reinterpret_cast<const f4*>(Gj + (wv * TRT + t) * 16 + acc_row(0));
+    // DOE consecutive columns of one token per thread: one vector load (past
+    // the end, of the last token, dropped where it is used)
     const int c = tid / (BV / DOE), vl = (tid % (BV / DOE)) * DOE, t = j * M + c;
-    if (t < a.T) {
-      o.dor = *reinterpret_cast<const DV*>(dob + (size_t)t * H * V + v0 + vl);
-      o.dm = mixb[(size_t)t * H * a.L];
-    } else {
-      o.dor = DV{};
-      o.dm = E(0.f);
-    }
-    o.has_add = a.inj && (j + 1) % a.inj_every == 0 && (j + 1) / a.inj_every <= a.inj_nf;
-    if (o.has_add) read_kv(a.inj + ((size_t)bh * a.inj_nf + (j + 1) / a.inj_every - 1) * K * V, o.add);
+    o.live = t < a.T;
+    const size_t tc = o.live ? t : a.T - 1;
+    o.dor = *reinterpret_cast<const DV*>(dob + tc * H * V + v0 + vl);
+    if constexpr (BF) o.dm = reinterpret_cast<const unsigned short*>(mixb)[tc * H * a.L];
+    else o.dm = reinterpret_cast<const int*>(mixb)[tc * H * a.L];
   };
   // the operand fragments of the current step
   auto f_kt = [&](const Ops& o, int s) -> SF {
@@ -531,21 +550,19 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       const int m0 = wv * 16 + acc_row(0), vl = ct * 16 + acc_col();
-      if (a.dVn) {
+      if (!FUSED && a.dVn) {
         float* o = a.dVn + ((size_t)bh * S + jj) * M * V + (size_t)m0 * V + v0 + vl;
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[(size_t)r * V] = pdv[ct][r];
       }
-      if (a.dVnT)
+      if (FUSED || a.dVnT)
         *reinterpret_cast<f4*>(a.dVnT + (((size_t)bh * S + jj) * V + v0 + vl) * M + m0) = pdv[ct];
     }
   };
 
-  Ops nxt;
-  // steps [j0, j1) in reverse, from the state gradient after step j1 - 1
-  const int j0 = a.j0, j1 = a.j1 > 0 ? a.j1 : S;
-  if (j1 > j0) load(j1 - 1, nxt);
-  for (int j = j1 - 1; j >= j0; --j) {
+  // One step with its operands loaded: cur, and (bf16) pre; the step's own
+  // successor is loaded into nxt and pre.
+  auto step = [&](int j, int jn, const Ops& cur, Ops& nxt) {
     // ---- this step's slices into the wave's region (bf16; the previous
     // step's reads of the region were issued before, in this wave's order)
     if constexpr (BF) {
@@ -554,16 +571,15 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
       CW::store(oW, pre + 2 * (CK::NL + CQ::NL));
       CW::store(oG, pre + 2 * (CK::NL + CQ::NL + CW::NL));
     }
-    const Ops cur = nxt;
     if (cur.has_add) {
 #pragma unroll
       for (int i = 0; i < TPW; ++i) ds[i] += cur.add[i];
     }
 
-    // ---- the next step's operand loads (the last step reloads its own, so
-    // that no branch guards them); this step's dS' and dVn are stored after
-    // its dVn products, while those loads are in flight
-    load(j > j0 ? j - 1 : j0, nxt);
+    // ---- the next step's operand loads; this step's dS' and dVn are stored
+    // after its dVn products, while those loads are in flight
+    load(jn, nxt);
+    __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step
 
     // ---- dS' and mix_0 dO staged (transposed) as B operands
 #pragma unroll
@@ -574,9 +590,13 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
     }
     {
       const int c = tid / (BV / DOE), vl = (tid % (BV / DOE)) * DOE;
-      const float m = to_f(cur.dm);
+      float m;
+      if constexpr (BF) m = to_f(__builtin_bit_cast(bf16, (unsigned short)cur.dm));
+      else m = __builtin_bit_cast(float, cur.dm);
+      const DE x = __builtin_bit_cast(DE, cur.dor);
 #pragma unroll
-      for (int q = 0; q < DOE; ++q) sdO.put1((vl + q) * LDS_VN + c, to_f(cur.dor[q]) * m);
+      for (int q = 0; q < DOE; ++q)
+        sdO.put1((vl + q) * LDS_VN + c, cur.live ? to_f(x[q]) * m : 0.f);
     }
     lds_barrier();
 
@@ -639,6 +659,29 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
     }
     // s_dot and s_dvn are rewritten by the next step
     lds_barrier();
+  };
+  // steps [j0, j1) in reverse, from the state gradient after step j1 - 1; the
+  // operand sets alternate (see the upper levels' scan), and the last step
+  // loads its own again, so that no branch guards the loads
+  const int j0 = a.j0, j1 = a.j1 > 0 ? a.j1 : S;
+  if constexpr (!BF && K == 128 && BV == 32) {
+    // two sets would not fit the registers
+    Ops nxt;
+    if (j1 > j0) load(j1 - 1, nxt);
+    for (int j = j1 - 1; j >= j0; --j) {
+      const Ops cur = nxt;
+      step(j, j > j0 ? j - 1 : j0, cur, nxt);
+    }
+  } else {
+    Ops x, y;
+    if (j1 > j0) load(j1 - 1, x);
+    wait_global();
+    int j = j1 - 1;
+    for (; j > j0; j -= 2) {
+      step(j, j - 1, x, y);
+      step(j - 1, j - 2 >= j0 ? j - 2 : j - 1, y, x);
+    }
+    if (j == j0) step(j0, j0, x, y);
   }
   if (a.dinit) {
 #pragma unroll
@@ -662,7 +705,10 @@ static hipError_t launch_scan_bwd_bv(const ScanBwdArgs& a, hipStream_t st) {
     if constexpr (M == CH) {
       if (a.frag != (BF ? 3 : 0) || !a.W || !a.KtT || !a.Aqk || !a.dout || !a.mix)
         return hipErrorInvalidValue;
-      hipLaunchKernelGGL((scan_bwd_l0_kernel<E, K, BV>), dim3(grid), dim3(256), 0, st, a);
+      if (a.dVnT && !a.dVn)
+        hipLaunchKernelGGL((scan_bwd_l0_kernel<E, K, BV, true>), dim3(grid), dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((scan_bwd_l0_kernel<E, K, BV, false>), dim3(grid), dim3(256), 0, st, a);
       return hipGetLastError();
     }
     return hipErrorInvalidValue;
@@ -678,11 +724,8 @@ static hipError_t launch_scan_bwd_bv(const ScanBwdArgs& a, hipStream_t st) {
 
 template <typename E, int K, int M>
 static hipError_t launch_scan_bwd(const ScanBwdArgs& a, hipStream_t st) {
-  // few (batch, head) pairs: the bf16 reverse scans take 16-column slices,
-  // as the forward scans do
-  if constexpr (std::is_same<E, bf16>::value) {
-    if (a.B * a.H * (a.V / SCAN_BV) <= SCAN_NARROW_GRID) return launch_scan_bwd_bv<E, K, M, 16>(a, st);
-  }
+  // few (batch, head) pairs: 16-column slices, as the forward scans take
+  if (a.B * a.H * (a.V / SCAN_BV) <= SCAN_NARROW_GRID) return launch_scan_bwd_bv<E, K, M, 16>(a, st);
   return launch_scan_bwd_bv<E, K, M, SCAN_BV>(a, st);
 }
 
