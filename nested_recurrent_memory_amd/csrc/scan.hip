@@ -117,48 +117,70 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
     ct = p % CT;
     return true;
   };
-  auto load = [&](int j, Ops& o) {
-    const SplitTile<E> Aj = split_at<E>(Ab + (size_t)j * M * K, M * K);
-    const float* Uj = Ub + (size_t)j * M * V;
-    const SplitTile<E> Bj = split_at<E>(Bb + (size_t)j * K * M, K * M);
-    const float* Gj = Gb + (size_t)j * K;
+  // The loads of step j's operands in the order in which the step needs them:
+  // part 0, A; 1, Qg; 2, U; 3, Aqk; 4, BT and gam.
+  auto load = [&](auto part_c, int j, Ops& o) {
+    constexpr int PART = decltype(part_c)::value;
+    if constexpr (PART < 4) {
+      const SplitTile<E> Aj = split_at<E>(Ab + (size_t)j * M * K, M * K);
+      const SplitTile<E> Qj = split_at<E>(a.Qg + ((size_t)bh * S + j) * M * K, M * K);
+      const SplitTile<E> Pj = split_at<E>(a.Aqk + ((size_t)bh * S + j) * M * M, M * M);
+      const float* Uj = Ub + (size_t)j * M * V;
 #pragma unroll
-    for (int p = 0; p < NVP; ++p) {
-      int rt, ct;
-      if (vn_tile(p, rt, ct)) {
+      for (int p = 0; p < NVP; ++p) {
+        int rt, ct;
+        if (!vn_tile(p, rt, ct)) continue;
+        const int q = ONE_RT ? 0 : p / CT;
+        const int arow = (rt * 16 + (lane & 15)) * K + kofs<E>(lane);
+        const int prow = (rt * 16 + (lane & 15)) * M + kofs<E>(lane);
         if (ONE_RT ? p == 0 : p % CT == 0) {
-          const int arow = (rt * 16 + (lane & 15)) * K + kofs<E>(lane);
+          if constexpr (PART == 0) {
 #pragma unroll
-          for (int s = 0; s < NSK; ++s)
-            o.a[ONE_RT ? 0 : p / CT][s] = Aj.get(FRA ? frag_at(rt, s, K) : arow + s * KS);
-          if constexpr (OUT) {
-            const SplitTile<E> Qj = split_at<E>(a.Qg + ((size_t)bh * S + j) * M * K, M * K);
-            const SplitTile<E> Pj = split_at<E>(a.Aqk + ((size_t)bh * S + j) * M * M, M * M);
-            const int prow = (rt * 16 + (lane & 15)) * M + kofs<E>(lane);
+            for (int s = 0; s < NSK; ++s) o.a[q][s] = Aj.get(FRA ? frag_at(rt, s, K) : arow + s * KS);
+          }
+          if constexpr (PART == 1 && OUT) {
 #pragma unroll
-            for (int s = 0; s < NSK; ++s)
-              o.qg[ONE_RT ? 0 : p / CT][s] = Qj.get(FRA ? frag_at(rt, s, K) : arow + s * KS);
+            for (int s = 0; s < NSK; ++s) o.qg[q][s] = Qj.get(FRA ? frag_at(rt, s, K) : arow + s * KS);
+          }
+          if constexpr (PART == 3 && OUT) {
 #pragma unroll
-            for (int s = 0; s < NSM; ++s)
-              o.aq[ONE_RT ? 0 : p / CT][s] = Pj.get(FRA ? frag_at(rt, s, M) : prow + s * KS);
+            for (int s = 0; s < NSM; ++s) o.aq[q][s] = Pj.get(FRA ? frag_at(rt, s, M) : prow + s * KS);
           }
         }
+        if constexpr (PART == 2) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          o.u[p][r] = Uj[(size_t)(rt * 16 + acc_row(r)) * V + v0 + ct * 16 + acc_col()];
+          for (int r = 0; r < 4; ++r)
+            o.u[p][r] = Uj[(size_t)(rt * 16 + acc_row(r)) * V + v0 + ct * 16 + acc_col()];
+        }
+      }
+    } else {
+      const SplitTile<E> Bj = split_at<E>(Bb + (size_t)j * K * M, K * M);
+      const float* Gj = Gb + (size_t)j * K;
+#pragma unroll
+      for (int t = 0; t < TRT; ++t) {
+        const int rt = (wv * TPW) / CT + t;
+        const int brow = (rt * 16 + (lane & 15)) * M + kofs<E>(lane);
+#pragma unroll
+        for (int s = 0; s < NSM; ++s)
+          o.bt[t][s] = FRB ? Bj.get(frag_at(rt, s, M))
+                          : (!PADM || s * KS + kofs<E>(lane) < M) ? Bj.get(brow + s * KS)
+                                                                  : Mma<E>::szero();
+        o.g[t] = *reinterpret_cast<const f4*>(Gj + rt * 16 + acc_row(0));
       }
     }
-#pragma unroll
-    for (int t = 0; t < TRT; ++t) {
-      const int rt = (wv * TPW) / CT + t;
-      const int brow = (rt * 16 + (lane & 15)) * M + kofs<E>(lane);
-#pragma unroll
-      for (int s = 0; s < NSM; ++s)
-        o.bt[t][s] = FRB ? Bj.get(frag_at(rt, s, M))
-                        : (!PADM || s * KS + kofs<E>(lane) < M) ? Bj.get(brow + s * KS)
-                                                                : Mma<E>::szero();
-      o.g[t] = *reinterpret_cast<const f4*>(Gj + rt * 16 + acc_row(0));
-    }
+    __builtin_amdgcn_sched_barrier(0);   // the loads stay where the step places them
+  };
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+  using P2 = std::integral_constant<int, 2>;
+  using P3 = std::integral_constant<int, 3>;
+  using P4 = std::integral_constant<int, 4>;
+  auto load_all = [&](int j, Ops& o) {
+    load(P0{}, j, o);
+    load(P1{}, j, o);
+    load(P2{}, j, o);
+    load(P3{}, j, o);
+    load(P4{}, j, o);
   };
 
   // SM: the next step whose transposed state is due
@@ -166,8 +188,7 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
   int vk_next = SM ? (a.j0 + vk_step - 1) / vk_step * vk_step : 0;
   auto store_state = [&](int j) {
     // (SM: the mode is known, so no branch stands between a product and the
-    // stores of its result: across one, this compiler left out the wait
-    // states that an MFMA's result needs before it is read)
+    // stores of its result)
     const bool by_chunk = SM == 0 ? a.state_mode == 0 : SM < 3;
     const size_t base = (by_chunk ? (size_t)bh * S + j
                                   : ((size_t)b * a.NG + j) * H + h) * K * V;
@@ -248,8 +269,14 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
     }
   };
 
-  // One step with its operands already loaded.
-  auto step = [&](int j, const Ops& cur) {
+  // One step with its operands already loaded, placing the loads of step jn's
+  // operands between its phases: a wave that issues them all at once (28 KB)
+  // stands at the memory pipe, which takes 64 bytes per clock from the four
+  // waves, before it starts on the step (B H = 64, T = 8192, K = 128: 606 ->
+  // 555 us; B H = 16, T = 16384 without a backward: 629 -> 561 us, where a
+  // timing copy without loads takes 200 us and the loads alone 300 us).
+  auto step = [&](int j, const Ops& cur, int jn, Ops& nxt) {
+      load(P0{}, jn, nxt);
       // ---- the state, transposed, to LDS
 #pragma unroll
       for (int i = 0; i < TPW; ++i) {
@@ -260,71 +287,95 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
       lds_barrier();
 
       // ---- Vn = U - A S (and, OUT, the read's Qg S on the same tiles)
+      constexpr int CTV = ONE_RT ? NVP : CT;     // column tiles this wave's Vn tiles use
+      auto vn_ct = [&](int c) { return ONE_RT ? (wv + NWV * c) / RTV : c; };
       f4 rd[OUT ? NVP : 1];
+      {
+        SF fb[CTV][NSK];
 #pragma unroll
-      for (int p = 0; p < NVP; ++p) {
-        int rt, ct;
-        if (vn_tile(p, rt, ct)) {
-          f4 acc = f4_zero();
-          if constexpr (OUT) rd[p] = f4_zero();
-          const int brow = (ct * 16 + (lane & 15)) * LDS_ST + kofs<E>(lane);
+        for (int c = 0; c < CTV; ++c) {
+          const int brow = (vn_ct(c) * 16 + (lane & 15)) * LDS_ST + kofs<E>(lane);
 #pragma unroll
-          for (int s = 0; s < NSK; ++s) {
-            const auto fb = sST.get(brow + s * KS);
-            acc = Mma<E>::mma(acc, cur.a[ONE_RT ? 0 : p / CT][s], fb);
-            if constexpr (OUT) {
-              rd[p] = Mma<E>::mma(rd[p], cur.qg[ONE_RT ? 0 : p / CT][s], fb);
-            }
-          }
-          const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-          f4 vn;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) vn[r] = cur.u[p][r] - acc[r];
-          sVn.put4(vl * LDS_VN + m0, vn);
-          pvn[p] = vn;
+          for (int s = 0; s < NSK; ++s) fb[c][s] = sST.get(brow + s * KS);
         }
-      }
-      lds_barrier();
-
-      // ---- OUT: read0 = Qg S + Aqk Vn for the chunk's rows in the sequence
-      if constexpr (OUT) {
+        load(P1{}, jn, nxt);
 #pragma unroll
         for (int p = 0; p < NVP; ++p) {
           int rt, ct;
           if (vn_tile(p, rt, ct)) {
-            const int brow = (ct * 16 + (lane & 15)) * LDS_VN + kofs<E>(lane);
+            const int c = ONE_RT ? p : p % CT;
+            f4 acc = f4_zero();
+            if constexpr (OUT) rd[p] = f4_zero();
 #pragma unroll
-            for (int s = 0; s < NSM; ++s) {
-              rd[p] = Mma<E>::mma(rd[p], cur.aq[ONE_RT ? 0 : p / CT][s], sVn.get(brow + s * KS));
+            for (int s = 0; s < NSK; ++s) {
+              acc = Mma<E>::mma(acc, cur.a[ONE_RT ? 0 : p / CT][s], fb[c][s]);
+              if constexpr (OUT) rd[p] = Mma<E>::mma(rd[p], cur.qg[ONE_RT ? 0 : p / CT][s], fb[c][s]);
             }
-            prd[p] = rd[p];
+            const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
+            f4 vn;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) vn[r] = cur.u[p][r] - acc[r];
+            sVn.put4(vl * LDS_VN + m0, vn);
+            pvn[p] = vn;
           }
         }
       }
-      // ---- this step's stores (the state registers still hold the state
-      // entering step j)
-      store_state(j);
-      flush(j);
+      load(P2{}, jn, nxt);
+      lds_barrier();
 
-      // ---- S <- diag(gam) S + BT Vn
+      // ---- Vn^T of every column tile, once for the read and the state
+      SF fv[CT][NSM];
 #pragma unroll
-      for (int i = 0; i < TPW; ++i) {
-        // t must be a compile-time index into the operand registers
-        constexpr bool WHOLE = TPW % CT == 0;
-        const int t = WHOLE ? i / CT : 0;
-        const int ct = WHOLE ? i % CT : (wv * TPW + i) % CT;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) st[i][r] *= cur.g[t][r];
-        const int brow = (ct * 16 + (lane & 15)) * LDS_VN + kofs<E>(lane);
+      for (int c = 0; c < CT; ++c) {
+        const int brow = (c * 16 + (lane & 15)) * LDS_VN + kofs<E>(lane);
 #pragma unroll
         for (int s = 0; s < NSM; ++s) {
           // M = 16 with 32-deep bf16 MFMAs: the upper half of the k range is zero
           const bool live = !PADM || (s * KS + kofs<E>(lane) < M);
-          typename Mma<E>::SFrag fb = Mma<E>::szero();
-          if (live) fb = sVn.get(brow + s * KS);
-          st[i] = Mma<E>::mma(st[i], cur.bt[t][s], fb);
+          fv[c][s] = Mma<E>::szero();
+          if (live) fv[c][s] = sVn.get(brow + s * KS);
         }
       }
+      // ---- OUT: read0 = Qg S + Aqk Vn for the chunk's rows in the sequence
+      if constexpr (OUT) {
+        static_assert(!OUT || (ONE_RT && RTV == NWV), "one row tile per wave, column tile p");
+#pragma unroll
+        for (int p = 0; p < NVP; ++p) {
+#pragma unroll
+          for (int s = 0; s < NSM; ++s) rd[p] = Mma<E>::mma(rd[p], cur.aq[0][s], fv[p][s]);
+          prd[p] = rd[p];
+        }
+      }
+      load(P3{}, jn, nxt);
+      // ---- this step's stores (the state registers still hold the state
+      // entering step j)
+      store_state(j);
+      flush(j);
+      load(P4{}, jn, nxt);
+
+      // ---- S <- diag(gam) S + BT Vn
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        // t and the column tile must be compile-time indices into registers
+        constexpr bool WHOLE = TPW % CT == 0;
+        const int t = WHOLE ? i / CT : 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) st[i][r] *= cur.g[t][r];
+        const int ct = WHOLE ? i % CT : (wv * TPW + i) % CT;
+#pragma unroll
+        for (int s = 0; s < NSM; ++s) {
+          if constexpr (WHOLE) {
+            st[i] = Mma<E>::mma(st[i], cur.bt[t][s], fv[i % CT][s]);
+          } else {
+            SF fb = fv[0][s];
+#pragma unroll
+            for (int c = 1; c < CT; ++c)
+              if (ct == c) fb = fv[c][s];
+            st[i] = Mma<E>::mma(st[i], cur.bt[t][s], fb);
+          }
+        }
+      }
+    mfma_settle();
     // no barrier needed here: the next writes to s_st do not alias s_vn, and
     // the next writes to s_vn follow the next step's barrier
   };
@@ -333,27 +384,23 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
   // j0. Each step's operand loads are issued a step ahead, unconditionally (the
   // last step reloads its own, so that no branch guards them).
   const int j0 = a.j0, j1 = a.j1 > 0 ? a.j1 : S;
-  if constexpr (SM != 0) {
+  // (128 pairs at K = 128 in 32 columns: two sets would not fit the registers)
+  if constexpr (SM != 0 && !(K == 128 && M == 128 && BV == 32)) {
     Ops x, y;
-    if (j1 > j0) load(j0, x);
+    if (j1 > j0) load_all(j0, x);
     wait_global();
     int j = j0;
     for (; j + 1 < j1; j += 2) {
-      load(j + 1, y);
-      __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step
-      step(j, x);
-      load(j + 2 < j1 ? j + 2 : j + 1, x);
-      __builtin_amdgcn_sched_barrier(0);
-      step(j + 1, y);
+      step(j, x, j + 1, y);
+      step(j + 1, y, j + 2 < j1 ? j + 2 : j + 1, x);
     }
-    if (j < j1) step(j, x);
+    if (j < j1) step(j, x, j, y);
   } else {
     Ops nxt;
-    if (j1 > j0) load(j0, nxt);
+    if (j1 > j0) load_all(j0, nxt);
     for (int j = j0; j < j1; ++j) {
       const Ops cur = nxt;
-      load(j + 1 < j1 ? j + 1 : j, nxt);
-      step(j, cur);
+      step(j, cur, j + 1 < j1 ? j + 1 : j, nxt);
     }
   }
   if (a.state_mode == 1 && j1 == S) {

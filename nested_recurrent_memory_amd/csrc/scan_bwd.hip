@@ -124,10 +124,10 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
     bool has_inj;
   };
   constexpr bool ALLV = RTV % 4 == 0;          // every wave has all its dVn tiles
-  auto load = [&](int j, Ops& o) {
+  // the operands of the dVn products, and those of the dS products: the step
+  // places the two parts apart (see scan.hip)
+  auto load_v = [&](int j, Ops& o) {
     const SplitTile<E> Bj = split_at<E>(Bb + (size_t)j * M * K, M * K);
-    const SplitTile<E> Aj = split_at<E>(Ab + (size_t)j * K * M, K * M);
-    const float* Gj = Gb + (size_t)j * K;
     const float* ip = inj_tile(j);
     o.has_inj = ip != nullptr;
     if (o.has_inj) read_kv(ip, o.inj);
@@ -140,6 +140,11 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
         for (int s = 0; s < NSK; ++s) o.bop[p][s] = Bj.get(brow + s * KS);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load_s = [&](int j, Ops& o) {
+    const SplitTile<E> Aj = split_at<E>(Ab + (size_t)j * K * M, K * M);
+    const float* Gj = Gb + (size_t)j * K;
 #pragma unroll
     for (int t = 0; t < TRT; ++t) {
       const int rt = (wv * TPW) / CT + t;
@@ -152,9 +157,11 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
       o.g[t] = *reinterpret_cast<const f4*>(Gj + rt * 16 + acc_row(0));
     }
     read_kv(dstates(j), o.add);
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  auto step = [&](int j, const Ops& cur) {
+  auto step = [&](int j, const Ops& cur, int jn, Ops& nxt) {
+    load_v(jn, nxt);
     // the group's read gradient and the injection into it (the branch stands
     // ahead of the products, not between one and the use of its result)
     f4 add[TPW];
@@ -192,14 +199,15 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
         }
       }
     }
+    load_s(jn, nxt);
     lds_barrier();
 
     // ---- dS' (the state gradient still holds it) and dVn to global
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int g = wv * TPW + i, rt = g / CT, ct = g % CT;
-      const int k0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-      float* o = a.dSp + ((size_t)bh * S + j) * K * V + (size_t)k0 * V + v0 + vl;
+      float* o = a.dSp + ((size_t)bh * S + j) * K * V + (size_t)(rt * 16 + acc_row(0)) * V + v0 +
+                 ct * 16 + acc_col();
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[(size_t)r * V] = ds[i][r];
     }
@@ -209,8 +217,8 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
       if (ALLV || rt < RTV) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-          const int m0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-          float* o = a.dVn + ((size_t)bh * S + j) * M * V + (size_t)m0 * V + v0 + vl;
+          float* o = a.dVn + ((size_t)bh * S + j) * M * V + (size_t)(rt * 16 + acc_row(0)) * V + v0 +
+                     ct * 16 + acc_col();
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[(size_t)r * V] = dv[p][ct][r];
         }
@@ -233,6 +241,7 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) ds[i][r] = cur.g[t][r] * ds[i][r] - acc[r] + add[i][r];
     }
+    mfma_settle();
     // no barrier here: the next step's writes of s_dst follow this step's
     // second barrier, after every read of s_dst, and its writes of s_dvn
     // follow the next step's first barrier, after every read of s_dvn
@@ -241,26 +250,27 @@ __global__ __launch_bounds__(256) void scan_bwd_kernel(ScanBwdArgs a) {
   if constexpr (K == 128 && M == 128) {
     // two sets would not fit the registers
     Ops nxt;
-    if (S > 0) load(S - 1, nxt);
+    if (S > 0) {
+      load_v(S - 1, nxt);
+      load_s(S - 1, nxt);
+    }
     for (int j = S - 1; j >= 0; --j) {
       const Ops cur = nxt;
-      load(j > 0 ? j - 1 : 0, nxt);
-      step(j, cur);
+      step(j, cur, j > 0 ? j - 1 : 0, nxt);
     }
   } else {
     Ops x, y;
-    if (S > 0) load(S - 1, x);
+    if (S > 0) {
+      load_v(S - 1, x);
+      load_s(S - 1, x);
+    }
     wait_global();
     int j = S - 1;
     for (; j > 0; j -= 2) {
-      load(j - 1, y);
-      __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step
-      step(j, x);
-      load(j > 1 ? j - 2 : 0, x);
-      __builtin_amdgcn_sched_barrier(0);
-      step(j - 1, y);
+      step(j, x, j - 1, y);
+      step(j - 1, y, j > 1 ? j - 2 : 0, x);
     }
-    if (j == 0) step(0, x);
+    if (j == 0) step(0, x, 0, y);
   }
   if (a.dinit) {
 #pragma unroll
@@ -414,8 +424,10 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
   // dS'^T, dVn^T and (mix_0 dO)^T, split once by their writers
   __shared__ __attribute__((aligned(16))) typename ST::T s_dst[ST::NPLANE * BV * LDS_ST];
   __shared__ __attribute__((aligned(16))) typename ST::T s_dvn[ST::NPLANE * BV * LDS_VN];
-  __shared__ __attribute__((aligned(16))) typename ST::T s_dot[ST::NPLANE * BV * LDS_VN];
-  const ST sdS{s_dst, BV * LDS_ST}, sdV{s_dvn, BV * LDS_VN}, sdO{s_dot, BV * LDS_VN};
+  // (dO in two buffers, used in turn: the next step stages its dO while this
+  // one's is still read, with no barrier between the steps)
+  __shared__ __attribute__((aligned(16))) typename ST::T s_dot[2][ST::NPLANE * BV * LDS_VN];
+  const ST sdS{s_dst, BV * LDS_ST}, sdV{s_dvn, BV * LDS_VN};
   // bf16: every wave's copy of its slices of KtT, Aqk, W and Qg
   using CK = SliceCopy<K, 16>;
   using CQ = SliceCopy<M, 16>;
@@ -482,25 +494,22 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
     bool has_add;
   };
   R16 pre[BF ? NSEG : 1];       // bf16: the next step's slice segments, raw
-  auto load = [&](int j, Ops& o) {
+  // The loads in two parts, placed apart by the step (see scan.hip): the
+  // operands of the dVn products with the token rows, and those of the dS
+  // products.
+  auto load_v = [&](int j, Ops& o) {
     o.has_add = a.inj && (j + 1) % a.inj_every == 0 && (j + 1) / a.inj_every <= a.inj_nf;
     if (o.has_add) read_kv(a.inj + ((size_t)bh * a.inj_nf + (j + 1) / a.inj_every - 1) * K * V, o.add);
     if constexpr (BF) {
       const bf16* kt = reinterpret_cast<const bf16*>(tile(a.KtT, j, K * M));
       const bf16* aq = reinterpret_cast<const bf16*>(tile(a.Aqk, j, M * M));
-      const bf16* wq = reinterpret_cast<const bf16*>(tile(a.W, j, M * K));
-      const bf16* qq = reinterpret_cast<const bf16*>(tile(a.Qg, j, M * K));
       CK::template load<M>(kt, 16 * wv, pre);
       CQ::template load<M>(aq, 16 * wv, pre + 2 * CK::NL);
-      CW::template load<K>(wq, NCW * wv, pre + 2 * (CK::NL + CQ::NL));
-      CW::template load<K>(qq, NCW * wv, pre + 2 * (CK::NL + CQ::NL + CW::NL));
     } else {
       // element e of a fragment (row tile rt of X^T, k = 16 s + 4 (lane / 16) + e)
       // = X[k][16 rt + lane % 16]
       const float* kt = tile(a.KtT, j, K * M);
       const float* aq = tile(a.Aqk, j, M * M);
-      const float* wq = tile(a.W, j, M * K);
-      const float* qq = tile(a.Qg, j, M * K);
       const int lr = 4 * (lane >> 4), lc = lane & 15;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -508,19 +517,8 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
         for (int s = 0; s < FK; ++s) o.kt[s][e] = kt[(16 * s + lr + e) * M + 16 * wv + lc];
 #pragma unroll
         for (int s = 0; s < FM; ++s) o.aq[s][e] = aq[(16 * s + lr + e) * M + 16 * wv + lc];
-#pragma unroll
-        for (int t = 0; t < FT; ++t)
-#pragma unroll
-          for (int s = 0; s < FM; ++s) {
-            o.wt[t][s][e] = wq[(16 * s + lr + e) * K + NCW * wv + 16 * t + lc];
-            o.qg[t][s][e] = qq[(16 * s + lr + e) * K + NCW * wv + 16 * t + lc];
-          }
       }
     }
-    const float* Gj = Gb + (size_t)j * K;
-#pragma unroll
-    for (int t = 0; t < TRT; ++t)
-      o.g[t] = *reinterpret_cast<const f4*>(Gj + (wv * TRT + t) * 16 + acc_row(0));
     // DOE consecutive columns of one token per thread: one vector load (past
     // the end, of the last token, dropped where it is used)
     const int c = tid / (BV / DOE), vl = (tid % (BV / DOE)) * DOE, t = j * M + c;
@@ -529,6 +527,33 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
     o.dor = *reinterpret_cast<const DV*>(dob + tc * H * V + v0 + vl);
     if constexpr (BF) o.dm = reinterpret_cast<const unsigned short*>(mixb)[tc * H * a.L];
     else o.dm = reinterpret_cast<const int*>(mixb)[tc * H * a.L];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load_s = [&](int j, Ops& o) {
+    if constexpr (BF) {
+      const bf16* wq = reinterpret_cast<const bf16*>(tile(a.W, j, M * K));
+      const bf16* qq = reinterpret_cast<const bf16*>(tile(a.Qg, j, M * K));
+      CW::template load<K>(wq, NCW * wv, pre + 2 * (CK::NL + CQ::NL));
+      CW::template load<K>(qq, NCW * wv, pre + 2 * (CK::NL + CQ::NL + CW::NL));
+    } else {
+      const float* wq = tile(a.W, j, M * K);
+      const float* qq = tile(a.Qg, j, M * K);
+      const int lr = 4 * (lane >> 4), lc = lane & 15;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < FT; ++t)
+#pragma unroll
+          for (int s = 0; s < FM; ++s) {
+            o.wt[t][s][e] = wq[(16 * s + lr + e) * K + NCW * wv + 16 * t + lc];
+            o.qg[t][s][e] = qq[(16 * s + lr + e) * K + NCW * wv + 16 * t + lc];
+          }
+    }
+    const float* Gj = Gb + (size_t)j * K;
+#pragma unroll
+    for (int t = 0; t < TRT; ++t)
+      o.g[t] = *reinterpret_cast<const f4*>(Gj + (wv * TRT + t) * 16 + acc_row(0));
+    __builtin_amdgcn_sched_barrier(0);
   };
   // the operand fragments of the current step
   auto f_kt = [&](const Ops& o, int s) -> SF {
@@ -561,25 +586,35 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
   };
 
   // One step with its operands loaded: cur, and (bf16) pre; the step's own
-  // successor is loaded into nxt and pre.
-  auto step = [&](int j, int jn, const Ops& cur, Ops& nxt) {
-    // ---- this step's slices into the wave's region (bf16; the previous
-    // step's reads of the region were issued before, in this wave's order)
+  // successor jn is loaded into nxt and pre. Each half of the slices goes to
+  // LDS and is loaded again just ahead of the products that read it, so that
+  // the LDS stores and the loads of one half run beside the products of the
+  // other (B H = 16, T = 4096, K = 128: 240 -> 213 us; K = 64, B H = 128, T =
+  // 2048: 117 -> 101 us). In 32 columns at K = 128 both halves go at the top:
+  // HBM's rate holds that shape, and its loads are then out earlier (B H =
+  // 64, T = 8192: 712 against 730 us). which: the dO buffer.
+  constexpr bool APART = K < 128 || BV < 32;
+  auto slices_s = [&](int jn, Ops& nxt) {
+    if constexpr (BF) {
+      CW::store(oW, pre + 2 * (CK::NL + CQ::NL));
+      CW::store(oG, pre + 2 * (CK::NL + CQ::NL + CW::NL));
+    }
+    load_s(jn, nxt);
+  };
+  auto step = [&](int j, int jn, const Ops& cur, Ops& nxt, int which) {
+    const ST sdO{s_dot[which], BV * LDS_VN};
+    // ---- the slices of the dVn products into the wave's region (bf16; the
+    // previous step's reads of it were issued before, in this wave's order)
     if constexpr (BF) {
       CK::store(oK, pre);
       CQ::store(oQ, pre + 2 * CK::NL);
-      CW::store(oW, pre + 2 * (CK::NL + CQ::NL));
-      CW::store(oG, pre + 2 * (CK::NL + CQ::NL + CW::NL));
     }
     if (cur.has_add) {
 #pragma unroll
       for (int i = 0; i < TPW; ++i) ds[i] += cur.add[i];
     }
-
-    // ---- the next step's operand loads; this step's dS' and dVn are stored
-    // after its dVn products, while those loads are in flight
-    load(jn, nxt);
-    __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step
+    load_v(jn, nxt);
+    if constexpr (!APART) slices_s(jn, nxt);
 
     // ---- dS' and mix_0 dO staged (transposed) as B operands
 #pragma unroll
@@ -621,14 +656,15 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
         pdv[ct] = acc;
       }
     }
+    if constexpr (APART) slices_s(jn, nxt);
     lds_barrier();
 
     // ---- dS' (the state gradient still holds it) and dVn to global
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int g = wv * TPW + i, rt = g / CT, ct = g % CT;
-      const int k0 = rt * 16 + acc_row(0), vl = ct * 16 + acc_col();
-      float* o = a.dSp + ((size_t)bh * S + j) * K * V + (size_t)k0 * V + v0 + vl;
+      float* o = a.dSp + ((size_t)bh * S + j) * K * V + (size_t)(rt * 16 + acc_row(0)) * V + v0 +
+                 ct * 16 + acc_col();
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[(size_t)r * V] = ds[i][r];
     }
@@ -657,8 +693,10 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
         for (int r = 0; r < 4; ++r) ds[i][r] = cur.g[t][r] * ds[i][r] - acc[r] + qacc[r];
       }
     }
-    // s_dot and s_dvn are rewritten by the next step
-    lds_barrier();
+    mfma_settle();
+    // no barrier here: the next step writes s_dst (read before this step's
+    // second barrier) and the other dO buffer (last read a step ago, before
+    // this step's barriers), and s_dvn after its own first barrier
   };
   // steps [j0, j1) in reverse, from the state gradient after step j1 - 1; the
   // operand sets alternate (see the upper levels' scan), and the last step
@@ -667,21 +705,27 @@ __global__ __launch_bounds__(256) void scan_bwd_l0_kernel(ScanBwdArgs a) {
   if constexpr (!BF && K == 128 && BV == 32) {
     // two sets would not fit the registers
     Ops nxt;
-    if (j1 > j0) load(j1 - 1, nxt);
+    if (j1 > j0) {
+      load_v(j1 - 1, nxt);
+      load_s(j1 - 1, nxt);
+    }
     for (int j = j1 - 1; j >= j0; --j) {
       const Ops cur = nxt;
-      step(j, j > j0 ? j - 1 : j0, cur, nxt);
+      step(j, j > j0 ? j - 1 : j0, cur, nxt, j & 1);
     }
   } else {
     Ops x, y;
-    if (j1 > j0) load(j1 - 1, x);
+    if (j1 > j0) {
+      load_v(j1 - 1, x);
+      load_s(j1 - 1, x);
+    }
     wait_global();
     int j = j1 - 1;
     for (; j > j0; j -= 2) {
-      step(j, j - 1, x, y);
-      step(j - 1, j - 2 >= j0 ? j - 2 : j - 1, y, x);
+      step(j, j - 1, x, y, 0);
+      step(j - 1, j - 2 >= j0 ? j - 2 : j - 1, y, x, 1);
     }
-    if (j == j0) step(j0, j0, x, y);
+    if (j == j0) step(j0, j0, x, y, 0);
   }
   if (a.dinit) {
 #pragma unroll
