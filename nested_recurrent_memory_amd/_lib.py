@@ -85,6 +85,7 @@ SIGNATURES = {
 _RESTYPES = {"ngdn_last_error": ctypes.c_char_p, "ngdn_arch": ctypes.c_char_p}
 
 _lib = None
+_fns = {}             # entry point name -> the loaded library's function
 
 
 class NgdnError(RuntimeError):
@@ -108,6 +109,7 @@ def lib():
         if so.ngdn_version() != VERSION:
             raise NgdnError(f"{LIB_PATH} implements interface version {so.ngdn_version()}, "
                             f"this package calls version {VERSION}: rebuild the library")
+        _fns.update({name: getattr(so, name) for name in SIGNATURES})
         _lib = so
     return _lib
 
@@ -125,35 +127,38 @@ def call(name, *args, tag=None, stream=None):
     ``tag`` names the call in TIMING (default: the entry point); ``stream``
     is the torch stream the call launches on when it is not the current one
     (the timing events go on that stream)."""
+    if _lib is None:
+        lib()
     if TIMING is not None:
         start = torch.cuda.Event(enable_timing=True)
         end = torch.cuda.Event(enable_timing=True)
         start.record(stream)
-        rc = getattr(lib(), name)(*args)
+        rc = _fns[name](*args)
         end.record(stream)
         if stream is not None and stream != torch.cuda.current_stream():
             SIDE.add(tag or name)
         TIMING.setdefault(tag or name, []).append((start, end))
     else:
-        rc = getattr(lib(), name)(*args)
+        rc = _fns[name](*args)
     if rc != 0:
         msg = lib().ngdn_last_error().decode()
         raise NgdnError(f"{name} failed ({rc}): {msg}")
 
 
+# Pointers are plain integers: the argument types convert them, and a ctypes
+# object per pointer cost more than the rest of a call.
+
 def ptr(t):
     """Device pointer of a tensor (or NULL for None)."""
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def ptr_of_stream(st):
-    return ctypes.c_void_p(st.cuda_stream)
+    return st.cuda_stream
 
 
 class GateArgs(ctypes.Structure):

@@ -27,6 +27,7 @@ Forward, per call (reference composition ops/chunk.py:159-304):
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -189,9 +190,150 @@ def _run_groups(B, dev, launch):
     return len(spans)
 
 
-def _rows(b0, nb):
-    """View of batch rows [b0, b0 + nb) of a batch-leading tensor (None stays None)."""
-    return lambda t: None if t is None else t[b0:b0 + nb]
+# ---------------------------------------------------------------- working memory
+#
+# The working buffers of a pass come from one allocation each (what the
+# backward reads again from the forward, and what only the pass itself needs),
+# and the kernels take addresses inside it: some forty tensors per pass cost
+# more host time than the launches at small shapes (K = 64, B = 2, T = 3000,
+# H = 8, four levels: 1.29 -> 0.70 ms per forward + backward, whose kernels take
+# 0.64; K = 64, B = 1, T = 333, H = 16, two levels, forward: 145 -> 70 us).
+# Where each buffer lies depends on the shapes alone and is worked out once per
+# configuration; addresses are formed anew in every call, from the allocation
+# as the call (or autograd, for the backward) hands it over.
+
+class _Layout:
+    """Buffers in one allocation: name -> (byte offset, bytes per batch row,
+    shape), 256-byte aligned; row 0 for buffers without a batch axis."""
+
+    def __init__(self):
+        self.at, self.bytes = {}, 0
+
+    def add(self, name, *shape, es=4, batched=True):
+        n = math.prod(shape) * es
+        self.at[name] = (self.bytes, n // shape[0] if batched else 0, shape)
+        self.bytes += -(-n // 256) * 256
+
+    def ptrs(self, base, b0=0):
+        """name -> address of batch row b0 in the allocation at ``base``."""
+        return {n: base + o + b0 * r for n, (o, r, _) in self.at.items()}
+
+
+def _arena(lay, dev):
+    return torch.empty(lay.bytes, device=dev, dtype=torch.uint8)
+
+
+@functools.lru_cache(maxsize=256)
+def _fwd_layout(B, T, H, L, K, V, NTF, nq, f, merge, train, fused_promotion, fused_l0, nmax, es):
+    """(kept, tmp, levels) of a forward: the buffers the backward reads (an
+    empty layout without one), the others, and per level (None for level 0)
+    its pairs per firing, firings, groups and form."""
+    NT = -(-T // 64)
+    kept, tmp = _Layout(), _Layout()
+    keep = kept.add if train else tmp.add
+    for n, shape in (("W", (64, K)), ("Qg", (64, K)), ("KtT", (K, 64)), ("Aqk", (64, 64)),
+                     ("gam", (K,))):
+        keep(n, B, H, NT, *shape)
+    # U only for the two-launch chunk backward (the fused one forms dA from Vn)
+    (tmp.add if fused_l0 else keep)("U", B, H, NT, 64, V)
+    # level 0's read of every token, formed by the level-0 scan while each
+    # chunk's state is on chip; the output pass adds the upper levels' reads
+    # and the mix (and the backward's dmix_0 reads it again)
+    keep("read0", B, T, H, V)
+    # the state entering each chunk, transposed: read by level 1's probes at
+    # every f1-th chunk only, so only those are written
+    if L > 1:
+        keep("hT", B, H, NT, V, K)
+    if train:
+        keep("TT", B, H, NT, 64, 64)
+        keep("h", B, H, NT, K, V)
+        keep("vn", B, H, NT, 64, V)
+    levels = [None] * L
+    for lvl in range(1, L):
+        nf, ng = n_firings(NTF, f[lvl]), n_groups(NT, f[lvl])
+        N = K if merge else nq[lvl - 1]
+        nf1 = max(nf, 1)
+        # one launch: probes and updates on chip; the backward's keys,
+        # (keys b e^g)^T and e^g only when training
+        chain = fused_promotion and _chain_ok(K, N, merge)
+        levels[lvl] = dict(N=N, nf=nf, ng=ng, chain=chain)
+        if not chain:
+            tmp.add(f"A{lvl}", B, H, nf1, N, K)
+            tmp.add(f"KT{lvl}", B, H, nf1, K, N)
+            tmp.add(f"U{lvl}", B, H, nf1, N, V)
+        if train or not chain:
+            keep(f"gam{lvl}", B, H, nf1, K)
+        if train:
+            keep(f"keys{lvl}", B, H, nf1, N, K)
+            keep(f"AT{lvl}", B, H, nf1, K, N)
+        # group states as rows and transposed
+        keep(f"states{lvl}", B, ng, H, K, V)
+        keep(f"statesT{lvl}", B, ng, H, V, K)
+    if L > 1:     # the parameters with their last two axes swapped
+        for n in ("bpT", "wpT", "gpT") + (("kpT",) if train else ()):
+            keep(n, L - 1, H, K, V, es=es, batched=False)
+        if train:
+            keep("bankT", L - 1, H, K, nmax, es=es, batched=False)
+    return kept, tmp, levels
+
+
+@functools.lru_cache(maxsize=256)
+def _bwd_layout(B, T, H, L, K, V, levels, merge, fused_l0, carry):
+    """The backward's working buffers; levels: (N, nf) per upper level."""
+    NT = -(-T // 64)
+    lay = _Layout()
+    for lvl in range(1, L):
+        N, nf, ng = levels[lvl - 1]
+        nfa = max(nf, 1)
+        lay.add(f"d_states{lvl}", B, ng, H, K, V)
+        lay.add(f"dSp{lvl}", B, H, nfa, K, V)
+        lay.add(f"dvn{lvl}", B, H, nfa, N, V)
+        for j in range(6):
+            lay.add(f"ws{lvl}_{j}", B, H, nfa, N, K)
+        if not merge:
+            lay.add(f"dbank{lvl}", B, H, nfa, N, K)
+        lay.add(f"inj{lvl}", B, H, nfa, K, V)
+    # per-slice partials of the parameter-gradient sums, shared by the levels
+    # (their sums run one after another on one stream)
+    if L > 1:
+        lay.add("parts", 4, H, _lib.PARAM_SPLIT, K, V, batched=False)
+    lay.add("dSp0", B, H, NT, K, V)
+    lay.add("dVnT0", B, H, NT, V, 64)
+    # dQg, dKt: the fused chunk backward's workspaces; the rest only for the
+    # two-launch form
+    lay.add("dQg", B, H, NT, 64, K)
+    lay.add("dKt", B, H, NT, 64, K)
+    if not fused_l0:
+        lay.add("dVn0", B, H, NT, 64, V)
+        lay.add("dWT", B, H, NT, K, 64)
+        lay.add("dAqk", B, H, NT, 64, 64)
+        lay.add("dgam", B, H, NT, K)
+    if carry:
+        lay.add("carry", B, H, L, K, V)
+    return lay
+
+
+def _row(t, b0):
+    """Address of batch row b0 of a contiguous batch-leading tensor (None stays None)."""
+    if t is None:
+        return None
+    return t.data_ptr() + b0 * t.stride(0) * t.element_size() if b0 else t.data_ptr()
+
+
+class _Saved(dict):
+    """What a forward hands to its backward: the tensors (inputs in the
+    working dtype, the kept allocation, the final state, the parameters) and
+    the configuration. A working buffer's name gives a view of it."""
+
+    def buffer(self, name):
+        o, _, shape = self["layout"].at[name]
+        flat = self["kept"][o:o + math.prod(shape) * 4].view(torch.float32)
+        return flat.view(shape)
+
+    def __missing__(self, name):
+        if name in ("states", "statesT"):
+            return [None] + [self.buffer(f"{name}{lvl}") for lvl in range(1, len(self["levels"]))]
+        return self.buffer(name)
 
 
 def _fire_chunks(T, fire_partial):
@@ -217,62 +359,38 @@ def _forward(q, k, v, g, b, w, mix, qb, kp, bp, wp, gp, nq, f, L, scale,
     q_, k_, v_, b_, w_, mix_ = (cvt(x) for x in (q, k, v, b, w, mix))
     g_ = g.to(torch.float32).contiguous()
     init_ = init.to(torch.float32).contiguous() if init is not None else None
-    e = lambda *s, dt=wd: torch.empty(*s, device=dev, dtype=dt)  # noqa: E731
-    # working tensors between the kernels are fp32 whatever the input dtype
-    f32 = lambda *s: e(*s, dt=torch.float32)  # noqa: E731
-    opt = lambda *s: f32(*s) if train else None  # noqa: E731
+    merge = promotion == "merge"
+    f, nq = tuple(f), tuple(nq)
+    params, nmax = (), 0
+    if L > 1:
+        params = _working_params(qb, kp, bp, wp, gp, wd)
+        nmax = params[0].shape[2]
 
     # everything is allocated here, on the current stream, before any launch
-    W, U, Qg = f32(B, H, NT, 64, K), f32(B, H, NT, 64, V), f32(B, H, NT, 64, K)
-    KtT, Aqk = f32(B, H, NT, K, 64), f32(B, H, NT, 64, 64)
-    gam = f32(B, H, NT, K)
-    TT = opt(B, H, NT, 64, 64)
-    # the state entering each chunk, transposed: read by level 1's probes at
-    # every f1-th chunk only, so only those are written
-    hT = f32(B, H, NT, V, K) if L > 1 else None
-    h_, vn_ = opt(B, H, NT, K, V), opt(B, H, NT, 64, V)
+    kept_lay, tmp_lay, levels = _fwd_layout(B, T, H, L, K, V, NTF, nq, f, merge, train,
+                                            FUSED_PROMOTION, FUSED_L0_BWD, nmax,
+                                            wd.itemsize)
+    kept = _arena(kept_lay, dev) if train else None
+    tmp = _arena(tmp_lay, dev)
     final = torch.empty(B, H, L, K, V, device=dev, dtype=torch.float32)
-    states = [None] * L       # group states as rows [B,NG,H,K,V]
-    statesT = [None] * L      # and transposed [B,NG,H,V,K]
-    levels = [None] * L
-    merge = promotion == "merge"
-    par = {}
+    o = torch.empty(B, T, H, V, device=dev, dtype=wd)
+    kept_base, tmp_base = (kept.data_ptr() if train else 0), tmp.data_ptr()
     if L > 1:
-        par = _params(qb, kp, bp, wp, gp, wd, train)
-    for lvl in range(1, L):
-        nf, ng = n_firings(NTF, f[lvl]), n_groups(NT, f[lvl])
-        N = K if merge else nq[lvl - 1]
-        nf1 = max(nf, 1)
-        if FUSED_PROMOTION and _chain_ok(K, N, merge):
-            # one launch: probes and updates on chip; the backward's keys,
-            # (keys b e^g)^T and e^g only when training
-            levels[lvl] = dict(N=N, nf=nf, ng=ng, chain=True, gam=opt(B, H, nf1, K),
-                               keys=opt(B, H, nf1, N, K), AT=opt(B, H, nf1, K, N))
-        else:
-            levels[lvl] = dict(N=N, nf=nf, ng=ng, chain=False, A=f32(B, H, nf1, N, K),
-                               KT=f32(B, H, nf1, K, N), U=f32(B, H, nf1, N, V),
-                               gam=f32(B, H, nf1, K), keys=opt(B, H, nf1, N, K),
-                               AT=opt(B, H, nf1, K, N))
-        states[lvl], statesT[lvl] = f32(B, ng, H, K, V), f32(B, ng, H, V, K)
-    o = e(B, T, H, V)
-    # level 0's read of every token, formed by the level-0 scan while each
-    # chunk's state is on chip; the output pass adds the upper levels' reads
-    # and the mix (and the backward's dmix_0 reads it again)
-    read0 = f32(B, T, H, V)
-    P = _lib.ptr
-
-    def param_grads(d, lvl, sp, st):
-        lv, wk = levels[lvl], work[lvl]
-        ws = wk["ws"]
-        _lib.call("ngdn_param_grads", ctypes.byref(d), lvl, int(merge), lv["N"], lv["nf"],
-                  *(P(x) for x in ws[:5]), P(wk["dbank"]), par["nmax"], P(dqb), P(dkp),
-                  P(dbp), P(dwp), P(dgp), P(parts), sp, tag=f"ngdn_param_grads.{lvl}",
-                  stream=st)
+        p0 = {**tmp_lay.ptrs(tmp_base), **kept_lay.ptrs(kept_base)}
+        bank, kp_, bp_, wp_, gp_ = params
+        _transpose_into([bp_, wp_, gp_] + ([kp_, bank] if train else []),
+                        [p0[n] for n in ("bpT", "wpT", "gpT")
+                         + (("kpT", "bankT") if train else ())])
+        bank_p, kp_p = bank.data_ptr(), kp_.data_ptr()
 
     def launch(b0, nb, st):
-        R = _rows(b0, nb)
-        sp = _lib.ptr_of_stream(st)
+        sp = st.cuda_stream
         d = _lib.dims(nb, T, H, L, K, V, code, scale, hold_partial=NTF < NT)
+        dp = ctypes.byref(d)
+        p = {**tmp_lay.ptrs(tmp_base, b0), **kept_lay.ptrs(kept_base, b0)}
+        get = p.get
+        xq, xk, xv, xg, xb, xw, xmix = (_row(x, b0) for x in (q_, k_, v_, g_, b_, w_, mix_))
+        xinit, xfin = _row(init_, b0), _row(final, b0)
         ranges = _l0_ranges(nb, H, V, NT, code) if nb == B else [(0, NT)]
         ts = _aux_streams(dev)[0] if len(ranges) > 1 else st
         if ts is not st:
@@ -281,9 +399,8 @@ def _forward(q, k, v, g, b, w, mix, qb, kp, bp, wp, gp, nq, f, L, scale,
         # them to one or two ranges ahead of the scan measured slower)
         ready = []
         for c0, n in ranges:
-            _lib.call("ngdn_l0_intra_fwd", ctypes.byref(d), *(P(R(x)) for x in (
-                q_, k_, v_, g_, b_, w_, W, U, KtT, Qg, Aqk, gam, TT)), c0, n,
-                _lib.ptr_of_stream(ts), stream=ts)
+            _lib.call("ngdn_l0_intra_fwd", dp, xq, xk, xv, xg, xb, xw, p["W"], p["U"], p["KtT"],
+                      p["Qg"], p["Aqk"], p["gam"], get("TT"), c0, n, ts.cuda_stream, stream=ts)
             ready.append(ts.record_event() if ts is not st else None)
         # with several ranges and unfused promotions, the upper levels follow
         # on a second side stream, one range behind: after level-0 range p,
@@ -291,25 +408,24 @@ def _forward(q, k, v, g, b, w, mix, qb, kp, bp, wp, gp, nq, f, L, scale,
         tu = (_aux_streams(dev)[1] if len(ranges) > 1 and L > 1
               and not any(levels[lvl]["chain"] for lvl in range(1, L)) else None)
         done = [0] * L          # firings of each level probed and scanned so far
-        for p, (c0, n) in enumerate(ranges):
-            if ready[p] is not None:
-                st.wait_event(ready[p])
+        for i, (c0, n) in enumerate(ranges):
+            if ready[i] is not None:
+                st.wait_event(ready[i])
             # a range after the first starts from the state the one before left in final
-            _lib.call("ngdn_l0_scan_fwd", ctypes.byref(d), *(P(R(x)) for x in (
-                W, U, KtT, gam, Qg, Aqk, init_ if p == 0 else final)), f[1] if L > 1 else 1,
-                *(P(R(x)) for x in (hT, None, h_, vn_, read0, final)), c0, n, sp)
+            _lib.call("ngdn_l0_scan_fwd", dp, p["W"], p["U"], p["KtT"], p["gam"], p["Qg"], p["Aqk"],
+                      xinit if i == 0 else xfin, f[1] if L > 1 else 1, get("hT"), None, get("h"),
+                      get("vn"), p["read0"], xfin, c0, n, sp)
             if tu is not None:
                 tu.wait_event(st.record_event())
-                upper_batch(d, R, done, c0 + n, p == len(ranges) - 1, tu)
+                upper_batch(dp, p, xinit, xfin, done, c0 + n, i == len(ranges) - 1, tu)
         if tu is not None:
             st.wait_event(tu.record_event())
         else:
-            upper_batch(d, R, done, NT, True, st)
-        spT, ngs, fs = _level_arrays([R(x) for x in statesT], NT, f, L)
-        _lib.call("ngdn_output_upper_fwd", ctypes.byref(d), P(R(read0)), P(R(q_)),
-                  P(R(mix_)), spT, ngs, fs, P(R(o)), sp)
+            upper_batch(dp, p, xinit, xfin, done, NT, True, st)
+        spT, ngs, fs = _level_arrays([None] + [p[f"statesT{lvl}"] for lvl in range(1, L)], NT, f, L)
+        _lib.call("ngdn_output_upper_fwd", dp, p["read0"], xq, xmix, spT, ngs, fs, _row(o, b0), sp)
 
-    def upper_batch(d, R, done, avail, last, su):
+    def upper_batch(dp, p, xinit, xfin, done, avail, last, su):
         """Probes and scans of every upper level for the firings whose lower
         state is stored: level 0 has stored the states entering chunks
         [0, avail); each level then has stored the groups entering its firings
@@ -317,39 +433,35 @@ def _forward(q, k, v, g, b, w, mix, qb, kp, bp, wp, gp, nq, f, L, scale,
         ((i + 1) f_here) / f_below, so the firings with (i + 1) f_here <
         avail f_below are ready; the last batch takes the rest (including
         those that read the lower final state) and stores every level's
-        trailing groups. d and R: the launch's dims and batch rows; su: the
+        trailing groups. dp, p: the launch's dims and addresses; su: the
         stream."""
-        sp = _lib.ptr_of_stream(su)
+        sp = su.cuda_stream
+        get = p.get
         for lvl in range(1, L):
             lv = levels[lvl]
             fh, fb = f[lvl], f[lvl - 1]
-            nf = lv["nf"]
+            nf, N = lv["nf"], lv["N"]
             upto = nf if last else min(nf, max(0, (avail * fb - 1) // fh))
             i0 = done[lvl]
             if lv["chain"]:
-                belowT, ngb = (hT, NT) if lvl == 1 else (statesT[lvl - 1], n_groups(NT, fb))
-                _lib.call("ngdn_promote_chain_fwd", ctypes.byref(d), lvl, int(merge), lv["N"], fb,
-                          fh, P(R(belowT)), ngb, P(R(final)), P(par["qb"]), par["nmax"],
-                          P(par["kp"]), P(par["bpT"]), P(par["wpT"]), P(par["gpT"]), P(R(init_)),
-                          P(R(states[lvl])), P(R(statesT[lvl])),
-                          *(P(R(lv[x])) for x in ("keys", "AT", "gam")), sp,
-                          tag=f"ngdn_promote_chain_fwd.{lvl}")
+                belowT, ngb = (p["hT"], NT) if lvl == 1 else (p[f"statesT{lvl - 1}"], n_groups(NT, fb))
+                _lib.call("ngdn_promote_chain_fwd", dp, lvl, int(merge), N, fb, fh, belowT, ngb, xfin,
+                          bank_p, nmax, kp_p, p["bpT"], p["wpT"], p["gpT"], xinit,
+                          p[f"states{lvl}"], p[f"statesT{lvl}"], get(f"keys{lvl}"), get(f"AT{lvl}"),
+                          get(f"gam{lvl}"), sp, tag=f"ngdn_promote_chain_fwd.{lvl}")
                 continue
-            below, ngb = (hT, NT) if lvl == 1 else (states[lvl - 1], n_groups(NT, fb))
+            below, ngb = (p["hT"], NT) if lvl == 1 else (p[f"states{lvl - 1}"], n_groups(NT, fb))
+            A, KT, U, gam = p[f"A{lvl}"], p[f"KT{lvl}"], p[f"U{lvl}"], p[f"gam{lvl}"]
             if upto > i0:
-                _lib.call("ngdn_probe_fwd", ctypes.byref(d), lvl, int(merge), lv["N"], fb, fh,
-                          P(R(below)), ngb, P(R(final)), P(par["qb"]), par["nmax"],
-                          P(par["kp"]), P(par["bpT"]), P(par["wpT"]), P(par["gpT"]),
-                          *(P(R(lv[x])) for x in ("A", "KT", "U", "gam", "keys", "AT")),
-                          None, None, None, None, None, i0, upto - i0, sp,
+                _lib.call("ngdn_probe_fwd", dp, lvl, int(merge), N, fb, fh, below, ngb, xfin, bank_p,
+                          nmax, kp_p, p["bpT"], p["wpT"], p["gpT"], A, KT, U, gam, get(f"keys{lvl}"),
+                          get(f"AT{lvl}"), None, None, None, None, None, i0, upto - i0, sp,
                           tag=f"ngdn_probe_fwd.{lvl}", stream=su)
             if upto > i0 or (last and nf == 0):
                 # a range after the level's first starts from the state in final
-                _lib.call("ngdn_upper_scan_fwd", ctypes.byref(d), lvl, lv["N"], nf, lv["ng"],
-                          *(P(R(lv[x])) for x in ("A", "KT", "U", "gam")),
-                          P(R(init_ if i0 == 0 else final)),
-                          P(R(states[lvl])), P(R(statesT[lvl])), P(R(final)), i0, upto - i0, sp,
-                          tag=f"ngdn_upper_scan_fwd.{lvl}", stream=su)
+                _lib.call("ngdn_upper_scan_fwd", dp, lvl, N, nf, lv["ng"], A, KT, U, gam,
+                          xinit if i0 == 0 else xfin, p[f"states{lvl}"], p[f"statesT{lvl}"], xfin, i0,
+                          upto - i0, sp, tag=f"ngdn_upper_scan_fwd.{lvl}", stream=su)
             done[lvl] = upto
             # the groups of this level stored so far bound the level above's firings
             avail = upto
@@ -357,35 +469,32 @@ def _forward(q, k, v, g, b, w, mix, qb, kp, bp, wp, gp, nq, f, L, scale,
     _run_groups(B, dev, launch)
     saved = None
     if train:
-        # U only for the two-launch chunk backward (the fused one forms dA
-        # from Vn instead)
-        saved = dict(q=q_, k=k_, v=v_, b=b_, w=w_, mix=mix_, g=g_, W=W,
-                     U=None if FUSED_L0_BWD else U, Qg=Qg,
-                     KtT=KtT, Aqk=Aqk, gam=gam, TT=TT, NTF=NTF,
-                     hT=hT, h=h_, vn=vn_, read0=read0, states=states,
-                     statesT=statesT, levels=levels, final=final, par=par,
-                     code=code, wd=wd)
+        saved = _Saved(q=q_, k=k_, v=v_, b=b_, w=w_, mix=mix_, g=g_, kept=kept, final=final,
+                       params=params, layout=kept_lay, levels=levels, fused_l0=FUSED_L0_BWD,
+                       NTF=NTF, code=code, wd=wd, nmax=nmax)
     return o, final, saved
 
 
-def _params(qb, kp, bp, wp, gp, wd, train):
-    """Per-level parameters in the layouts the kernels read: originals, the
-    projections with their last two axes swapped, and (for the backward) the
-    bank and key projections transposed. The bank is padded to a multiple of
-    8 rows so every row start is 16-byte aligned."""
+def _working_params(qb, kp, bp, wp, gp, wd):
+    """The parameters contiguous in the working dtype, the bank padded to a
+    multiple of 8 rows so every row start is 16-byte aligned. fp32 parameters
+    of a bf16 call (autocast) are cast in one launch."""
     nmax = qb.shape[2]
-    nmax8 = -(-nmax // 8) * 8
-    qb_ = qb.to(wd)
-    if nmax8 != nmax:
-        qb_ = torch.nn.functional.pad(qb_, (0, 0, 0, nmax8 - nmax))
-    c = lambda x: x.to(wd).contiguous()  # noqa: E731
-    qb_, kp_, bp_, wp_, gp_ = (c(x) for x in (qb_, kp, bp, wp, gp))
-    # the transposes in one launch
-    tr = _transpose_last2([bp_, wp_, gp_] + ([kp_, qb_] if train else []))
-    par = dict(qb=qb_, nmax=nmax8, kp=kp_, bpT=tr[0], wpT=tr[1], gpT=tr[2])
-    if train:
-        par.update(kpT=tr[3], bankT=tr[4], bp=bp_, wp=wp_, gp=gp_)
-    return par
+    if nmax % 8:
+        qb = torch.nn.functional.pad(qb, (0, 0, 0, -nmax % 8))
+    xs = [qb, kp, bp, wp, gp]
+    if wd == torch.bfloat16 and all(x.dtype == torch.float32 and x.is_contiguous() for x in xs):
+        return tuple(_cast_bf16(xs))
+    return tuple(x.to(wd).contiguous() for x in xs)
+
+
+def _params(qb, kp, bp, wp, gp, wd):
+    """Per-level parameters in the layouts the step's kernels read: the bank
+    and key projections as they are, the other projections with their last
+    two axes swapped."""
+    qb_, kp_, bp_, wp_, gp_ = _working_params(qb, kp, bp, wp, gp, wd)
+    tr = _transpose_last2([bp_, wp_, gp_])
+    return dict(qb=qb_, nmax=qb_.shape[2], kp=kp_, bpT=tr[0], wpT=tr[1], gpT=tr[2])
 
 
 def _transpose_last2(xs):
@@ -395,18 +504,38 @@ def _transpose_last2(xs):
         raise ValueError("_transpose_last2: contiguous tensors of one dtype, at least 2-D")
     outs = [torch.empty(x.shape[:-2] + (x.shape[-1], x.shape[-2]), device=x.device, dtype=x.dtype)
             for x in xs]
+    _transpose_into(xs, [y.data_ptr() for y in outs])
+    return outs
+
+
+def _transpose_into(xs, dsts):
+    """xs (contiguous, one dtype) transposed in their last two axes to the
+    addresses dsts, in one launch on the current stream."""
     n = len(xs)
-    _lib.call("ngdn_transpose", n, (ctypes.c_void_p * n)(*(x.data_ptr() for x in xs)),
-              (ctypes.c_void_p * n)(*(y.data_ptr() for y in outs)),
-              (ctypes.c_int32 * n)(*(x.numel() // max(1, x.shape[-1] * x.shape[-2]) for x in xs)),
-              (ctypes.c_int32 * n)(*(x.shape[-2] for x in xs)),
-              (ctypes.c_int32 * n)(*(x.shape[-1] for x in xs)),
+    I = ctypes.c_int32 * n  # noqa: E741
+    _lib.call("ngdn_transpose", n, (ctypes.c_void_p * n)(*[x.data_ptr() for x in xs]),
+              (ctypes.c_void_p * n)(*dsts),
+              I(*[x.numel() // max(1, x.shape[-1] * x.shape[-2]) for x in xs]),
+              I(*[x.shape[-2] for x in xs]), I(*[x.shape[-1] for x in xs]),
               xs[0].element_size(), _lib.stream_of(xs[0]))
+
+
+def _cast_bf16(xs):
+    """Contiguous fp32 tensors cast to bf16, each into a tensor of its own, in
+    one launch on the current stream."""
+    outs = [torch.empty(x.shape, device=x.device, dtype=torch.bfloat16) for x in xs]
+    n = len(xs)
+    _lib.call("ngdn_cast_bf16", n, (ctypes.c_void_p * n)(*[x.data_ptr() for x in xs]),
+              (ctypes.c_void_p * n)(*[y.data_ptr() for y in outs]),
+              (ctypes.c_int64 * n)(*[x.numel() for x in xs]), _lib.stream_of(xs[0]))
     return outs
 
 
 def _level_arrays(states, NT, f, L):
-    sp = (ctypes.c_void_p * L)(*([None] + [s.data_ptr() for s in states[1:]]))
+    """The per-level argument arrays of the output entry points; states:
+    tensors or addresses, the first (level 0) unused."""
+    sp = (ctypes.c_void_p * L)(*([None] + [s if isinstance(s, int) else s.data_ptr()
+                                           for s in states[1:]]))
     ngs = (ctypes.c_int32 * L)(*([0] + [n_groups(NT, f[l]) for l in range(1, L)]))
     fs = (ctypes.c_int32 * L)(*f)
     return sp, ngs, fs
@@ -419,84 +548,65 @@ def _backward(sv, do, dfinal, L, scale, f, nq, has_init, promotion):
     B, T, H, _, K = q_.shape
     V = v_.shape[-1]
     dev = q_.device
-    wd, code = sv["wd"], sv["code"]
+    wd, code, nmax = sv["wd"], sv["code"], sv["nmax"]
     NT = -(-T // 64)
-    P = _lib.ptr
     e = lambda *s, dt=wd: torch.empty(*s, device=dev, dtype=dt)  # noqa: E731
     f32 = lambda *s: e(*s, dt=torch.float32)  # noqa: E731
-    z32 = lambda *s: torch.zeros(*s, device=dev, dtype=torch.float32)  # noqa: E731
     do_ = do.to(wd).contiguous()
     merge = promotion == "merge"
-    states, levels, par, final = sv["states"], sv["levels"], sv["par"], sv["final"]
-
-    # everything is allocated (and zeroed) here, on the current stream; the
-    # buffers that start at zero share one allocation and one fill
-    zshapes = ([] if dfinal is not None else [(B, H, L, K, V)]) + \
-        ([(B, H, L, K, V)] if has_init else []) + \
-        ([(L - 1, H, par["nmax"], K), (L - 1, H, K, V), (L - 1, H, V, K), (L - 1, H, V, V),
-          (L - 1, H, V, K)] if L > 1 else [])
-    zsizes = [math.prod(sh) for sh in zshapes]
-    zbuf = z32(sum(zsizes)) if zshapes else None
-    zviews, off = [], 0
-    for sh, n in zip(zshapes, zsizes):
-        zviews.append(zbuf[off:off + n].view(sh))
-        off += n
-    zit = iter(zviews)
-    dq = e(B, T, H, L, K)
-    dmix = f32(B, T, H, L)
-    d_final = (dfinal.to(torch.float32).contiguous().clone() if dfinal is not None
-               else next(zit))
-    d_init = next(zit) if has_init else None
-    d_states = [None] + [f32(B, n_groups(NT, f[lvl]), H, K, V) for lvl in range(1, L)]
-    dqb = dkp = dbp = dwp = dgp = None
-    work = [None] * L
-    if L > 1:
-        dqb, dkp, dbp, dwp, dgp = (next(zit) for _ in range(5))
-    for lvl in range(1, L):
-        lv = levels[lvl]
-        N, nf = lv["N"], lv["nf"]
-        nfa = max(nf, 1)
-        work[lvl] = dict(dSp=f32(B, H, nfa, K, V), dvn=f32(B, H, nfa, N, V),
-                         ws=[f32(B, H, nfa, N, K) for _ in range(4)]
-                         + [f32(B, H, nfa, N, V) for _ in range(2)],
-                         dbank=None if merge else f32(B, H, nfa, N, K),
-                         inj=f32(B, H, nfa, K, V))
-    # per-slice partials of the parameter-gradient sums, shared by the levels
-    # (their sums run one after another on one stream)
-    parts = f32(4, H, _lib.PARAM_SPLIT, K, V) if L > 1 else None
-    dSp0, dVnT0 = f32(B, H, NT, K, V), f32(B, H, NT, V, 64)
-    # dQg, dKt: the fused chunk backward's workspaces; the rest only for the
-    # two-launch form
-    dQg, dKt = f32(B, H, NT, 64, K), f32(B, H, NT, 64, K)
-    dVn0 = dWT = dAqk = dgam = None
+    levels, final, params = sv["levels"], sv["final"], sv["params"]
     # the form the forward saved for (U is kept only for the two-launch form)
-    fused_l0 = sv["U"] is None
+    fused_l0 = sv["fused_l0"]
     # small grids, one group of rows, the fused chunk backward: the level-0
     # reverse scan runs the chunk ranges of the forward last first, the
-    # gradient of the state between ranges carried in l0_carry, and each
+    # gradient of the state between ranges carried in a buffer, and each
     # range's chunk backward runs on a side stream beside the scan of the
     # range before it
     l0_ranges = (_l0_ranges(B, H, V, NT, code)
                  if fused_l0 and max(1, min(STREAM_GROUPS, B)) == 1 else [(0, NT)])
-    l0_carry = f32(B, H, L, K, V) if len(l0_ranges) > 1 else None
-    if not fused_l0:
-        dVn0, dWT = f32(B, H, NT, 64, V), f32(B, H, NT, K, 64)
-        dAqk, dgam = f32(B, H, NT, 64, 64), f32(B, H, NT, K)
+
+    # everything is allocated (and zeroed) here, on the current stream
+    lay = _bwd_layout(B, T, H, L, K, V,
+                      tuple((lv["N"], lv["nf"], lv["ng"]) for lv in levels[1:]), merge, fused_l0,
+                      len(l0_ranges) > 1)
+    work = _arena(lay, dev)
+    work_base, kept_base, kept_lay = work.data_ptr(), sv["kept"].data_ptr(), sv["layout"]
+    dq, dmix = e(B, T, H, L, K), f32(B, T, H, L)
     dk, dv, db, dw = e(B, T, H, K), e(B, T, H, V), e(B, T, H, K), e(B, T, H, V)
     dg = f32(B, T, H, K)
+    zeros = []
+    if dfinal is not None:
+        d_final = dfinal.to(torch.float32).contiguous().clone()
+    else:
+        d_final = f32(B, H, L, K, V)
+        zeros.append(d_final)
+    d_init = f32(B, H, L, K, V) if has_init else None
+    if has_init:
+        zeros.append(d_init)
+    dqb = dkp = dbp = dwp = dgp = None
+    if L > 1:
+        dqb, dkp, dbp, dwp, dgp = (f32(L - 1, H, *s) for s in ((nmax, K), (K, V), (V, K), (V, V),
+                                                               (V, K)))
+        zeros += [dqb, dkp, dbp, dwp, dgp]
+        bank_p, kp_p, bp_p, wp_p, gp_p = (x.data_ptr() for x in params)
+        dpar = [x.data_ptr() for x in (dqb, dkp, dbp, dwp, dgp)]
+    if zeros:
+        torch._foreach_zero_(zeros)
 
-    def param_grads(d, lvl, sp, st):
-        lv, wk = levels[lvl], work[lvl]
-        ws = wk["ws"]
-        _lib.call("ngdn_param_grads", ctypes.byref(d), lvl, int(merge), lv["N"], lv["nf"],
-                  *(P(x) for x in ws[:5]), P(wk["dbank"]), par["nmax"], P(dqb), P(dkp),
-                  P(dbp), P(dwp), P(dgp), P(parts), sp, tag=f"ngdn_param_grads.{lvl}",
-                  stream=st)
+    def param_grads(dp, p, lvl, st):
+        lv = levels[lvl]
+        _lib.call("ngdn_param_grads", dp, lvl, int(merge), lv["N"], lv["nf"],
+                  *[p[f"ws{lvl}_{j}"] for j in range(5)], p.get(f"dbank{lvl}"), nmax, *dpar,
+                  p["parts"], st.cuda_stream, tag=f"ngdn_param_grads.{lvl}", stream=st)
 
     def launch(b0, nb, st):
-        R = _rows(b0, nb)
-        sp = _lib.ptr_of_stream(st)
+        sp = st.cuda_stream
         d = _lib.dims(nb, T, H, L, K, V, code, scale, hold_partial=sv["NTF"] < NT)
+        dp = ctypes.byref(d)
+        p = {**kept_lay.ptrs(kept_base, b0), **lay.ptrs(work_base, b0)}
+        get = p.get
+        xq, xk, xv, xg, xb, xw, xmix, xdo = (_row(x, b0) for x in (q_, k_, v_, g_, b_, w_, mix_, do_))
+        xfin, xdfin, xdinit, xdq, xdmix = (_row(x, b0) for x in (final, d_final, d_init, dq, dmix))
         # With one group of rows, independent launches go to two side streams:
         # (a) the reads' backward of the levels below the top one
         # (each writes its own columns of dmix and dq and its own d_states)
@@ -517,139 +627,105 @@ def _backward(sv, do, dfinal, L, scale, f, nq, has_init, promotion):
             for a in aux:
                 a.wait_event(fork)
         ta, tb = (aux[0], aux[1]) if aux else (st, st)
-        sa, sb = _lib.ptr_of_stream(ta), _lib.ptr_of_stream(tb)
         # reads: dmix for every level (level 0 from the stored read, on the
         # second side stream), dq and the group-state gradients for levels >= 1
         dmix0_done = []
 
         def dmix0():
-            _lib.call("ngdn_output_bwd", ctypes.byref(d), P(R(sv["read0"])), P(R(do_)),
-                      P(R(dmix)), sb, stream=tb)
+            _lib.call("ngdn_output_bwd", dp, p["read0"], xdo, xdmix, tb.cuda_stream, stream=tb)
             dmix0_done.append(True)
         if not (DMIX0_LATE and aux is not None):
             dmix0()
         late = READS_AFTER_TOP and aux is not None
         for lvl in ([L - 1] + list(range(1, L - 1)) if late else range(1, L)):
-            ng = n_groups(NT, f[lvl])
-            top = lvl == L - 1
-            _lib.call("ngdn_read_state_bwd", ctypes.byref(d), lvl, f[lvl], ng,
-                      *(P(R(x)) for x in (q_, mix_, do_, states[lvl], d_states[lvl], dq, dmix)),
-                      sp if top else sa, tag=f"ngdn_read_state_bwd.{lvl}", stream=st if top else ta)
-            if late and top:
-                aux[0].wait_stream(st)
+            t = st if lvl == L - 1 else ta
+            _lib.call("ngdn_read_state_bwd", dp, lvl, f[lvl], levels[lvl]["ng"], xq, xmix, xdo,
+                      p[f"states{lvl}"], p[f"d_states{lvl}"], xdq, xdmix, t.cuda_stream,
+                      tag=f"ngdn_read_state_bwd.{lvl}", stream=t)
+            if late and lvl == L - 1:
+                ta.wait_stream(st)
         joined = aux is None
         inj, nf1 = None, 0
         for lvl in range(L - 1, 0, -1):
-            lv, wk = levels[lvl], work[lvl]
+            lv = levels[lvl]
             N, nf, ng = lv["N"], lv["nf"], lv["ng"]
             if not joined and lvl < L - 1:
-                st.wait_stream(aux[0])
+                st.wait_stream(ta)
                 joined = True
             # the level above's injection (its probe backward's lower-state
             # gradients), added by this level's reverse scan
             up = lvl + 1 < L and levels[lvl + 1]["nf"] > 0
-            _lib.call("ngdn_upper_scan_bwd", ctypes.byref(d), lvl, N, nf, ng,
-                      *(P(R(x)) for x in (lv["keys"], lv["AT"], lv["gam"], d_states[lvl])),
-                      P(R(work[lvl + 1]["inj"])) if up else None, f[lvl],
-                      f[lvl + 1] if up else 1, levels[lvl + 1]["nf"] if up else 0,
-                      *(P(R(x)) for x in (d_final, wk["dSp"], wk["dvn"], d_init)),
-                      sp, tag=f"ngdn_upper_scan_bwd.{lvl}")
+            dSp, dvn, gam = p[f"dSp{lvl}"], p[f"dvn{lvl}"], get(f"gam{lvl}")
+            _lib.call("ngdn_upper_scan_bwd", dp, lvl, N, nf, ng, p[f"keys{lvl}"], p[f"AT{lvl}"], gam,
+                      p[f"d_states{lvl}"], p[f"inj{lvl + 1}"] if up else None, f[lvl],
+                      f[lvl + 1] if up else 1, levels[lvl + 1]["nf"] if up else 0, xdfin, dSp, dvn,
+                      xdinit, sp, tag=f"ngdn_upper_scan_bwd.{lvl}")
             if nf == 0:
                 continue
             fh, fb = f[lvl], f[lvl - 1]
             if lvl == 1:
-                inj, nf1 = wk["inj"], nf
-                b_kv, b_vk, ngb = sv["h"], sv["hT"], NT
+                inj, nf1 = p["inj1"], nf
+                b_kv, b_vk, ngb = p["h"], p["hT"], NT
             else:
-                b_kv, b_vk = states[lvl - 1], sv["statesT"][lvl - 1]
+                b_kv, b_vk = p[f"states{lvl - 1}"], p[f"statesT{lvl - 1}"]
                 ngb = n_groups(NT, fb)
-            ws = wk["ws"]
-            _lib.call("ngdn_probe_bwd", ctypes.byref(d), lvl, int(merge), N, fb, fh,
-                      P(R(b_kv)), P(R(b_vk)), ngb, P(R(final)), P(par["qb"]), par["nmax"],
-                      P(par["kp"]), P(par["bpT"]), P(par["wpT"]), P(par["gpT"]),
-                      P(par["kpT"]), P(par["bankT"]), P(par["bp"]), P(par["wp"]),
-                      P(par["gp"]), P(R(states[lvl])), P(R(sv["statesT"][lvl])), ng,
-                      P(R(wk["dSp"])), P(R(wk["dvn"])), *(P(R(x)) for x in ws),
-                      P(R(wk["dbank"])), P(R(wk["inj"])), P(R(d_final)), sp,
-                      tag=f"ngdn_probe_bwd.{lvl}")
+            _lib.call("ngdn_probe_bwd", dp, lvl, int(merge), N, fb, fh, b_kv, b_vk, ngb, xfin, bank_p,
+                      nmax, kp_p, p["bpT"], p["wpT"], p["gpT"], p["kpT"], p["bankT"], bp_p, wp_p, gp_p,
+                      p[f"states{lvl}"], p[f"statesT{lvl}"], ng, dSp, dvn,
+                      *[p[f"ws{lvl}_{j}"] for j in range(6)], get(f"dbank{lvl}"), p[f"inj{lvl}"],
+                      xdfin, sp, tag=f"ngdn_probe_bwd.{lvl}")
             if nb == B:
                 if aux is not None:
-                    aux[1].wait_stream(st)
+                    tb.wait_stream(st)
                 if DMIX0_LATE and aux is not None and lvl == 1:
                     dmix0()
-                param_grads(d, lvl, sb, tb)
+                param_grads(dp, p, lvl, tb)
         if not joined:
-            st.wait_stream(aux[0])
+            st.wait_stream(ta)
         if not dmix0_done:
             # (late placement) after the upper levels' parameter-gradient sums
             dmix0()
         # level 0
         ranges = l0_ranges if nb == B else [(0, NT)]
         tl = _aux_streams(dev)[0] if len(ranges) > 1 else st
-        for p in reversed(range(len(ranges))):
-            c0, n = ranges[p]
-            last = p == len(ranges) - 1
-            _lib.call("ngdn_l0_scan_bwd", ctypes.byref(d), *(P(R(sv[x])) for x in (
-                "W", "KtT", "gam", "Qg", "Aqk")), P(R(do_)), P(R(mix_)), f[1] if L > 1 else 1,
-                P(R(inj)), nf1, P(R(d_final if last else l0_carry)), P(R(dSp0)), P(R(dVn0)),
-                P(R(dVnT0)), P(R(d_init if p == 0 else l0_carry)), c0, n, sp)
+        xdk, xdv, xdg, xdb, xdw = (_row(x, b0) for x in (dk, dv, dg, db, dw))
+        for i in reversed(range(len(ranges))):
+            c0, n = ranges[i]
+            last = i == len(ranges) - 1
+            _lib.call("ngdn_l0_scan_bwd", dp, p["W"], p["KtT"], p["gam"], p["Qg"], p["Aqk"], xdo, xmix,
+                      f[1] if L > 1 else 1, inj, nf1, xdfin if last else p["carry"], p["dSp0"],
+                      get("dVn0"), p["dVnT0"], xdinit if i == 0 else p["carry"], c0, n, sp)
             if fused_l0:
                 # the chunk backward in one launch: the state half per chunk
                 if tl is not st:
                     tl.wait_event(st.record_event())
-                _lib.call("ngdn_l0_bwd", ctypes.byref(d), *(P(R(x)) for x in (
-                    q_, k_, v_, g_, b_, w_, sv["TT"], sv["h"], dSp0, sv["vn"],
-                    dVnT0, do_, mix_, dQg, dKt, dq, dk, dv, dg, db, dw)), c0, n,
-                    _lib.ptr_of_stream(tl), stream=tl)
+                _lib.call("ngdn_l0_bwd", dp, xq, xk, xv, xg, xb, xw, p["TT"], p["h"], p["dSp0"], p["vn"],
+                          p["dVnT0"], xdo, xmix, p["dQg"], p["dKt"], xdq, xdk, xdv, xdg, xdb, xdw, c0, n,
+                          tl.cuda_stream, stream=tl)
         if tl is not st:
             st.wait_stream(tl)
         if not fused_l0:
-            _lib.call("ngdn_l0_bwd_state", ctypes.byref(d), P(R(sv["h"])), P(R(dSp0)),
-                      P(R(sv["vn"])), P(R(dVn0)), P(R(do_)), P(R(mix_)),
-                      *(P(R(x)) for x in (dQg, dWT, dKt, dAqk, dgam)), sp)
-            _lib.call("ngdn_l0_bwd_intra", ctypes.byref(d), *(P(R(x)) for x in (
-                q_, k_, v_, g_, b_, w_, sv["W"], sv["U"], sv["TT"], dQg, dWT, dKt, dAqk, dgam,
-                dVnT0, dq, dk, dv, dg, db, dw)), sp)
+            _lib.call("ngdn_l0_bwd_state", dp, p["h"], p["dSp0"], p["vn"], p["dVn0"], xdo, xmix,
+                      p["dQg"], p["dWT"], p["dKt"], p["dAqk"], p["dgam"], sp)
+            _lib.call("ngdn_l0_bwd_intra", dp, xq, xk, xv, xg, xb, xw, p["W"], p["U"], p["TT"], p["dQg"],
+                      p["dWT"], p["dKt"], p["dAqk"], p["dgam"], p["dVnT0"], xdq, xdk, xdv, xdg, xdb, xdw,
+                      sp)
         if aux is not None:
-            st.wait_stream(aux[1])
+            st.wait_stream(tb)
 
     groups = _run_groups(B, dev, launch)
     if groups > 1:
         st = torch.cuda.current_stream(dev)
         d = _lib.dims(B, T, H, L, K, V, code, scale, hold_partial=sv["NTF"] < NT)
+        p = lay.ptrs(work_base)
         for lvl in range(L - 1, 0, -1):
             if levels[lvl]["nf"] > 0:
-                param_grads(d, lvl, _lib.ptr_of_stream(st), st)
+                param_grads(ctypes.byref(d), p, lvl, st)
     return dq, dk, dv, dg, db, dw, dmix, dqb, dkp, dbp, dwp, dgp, d_init
 
 
-def _flatten(x, tensors):
-    """x with every tensor replaced by its index in ``tensors`` (appended)."""
-    if isinstance(x, torch.Tensor):
-        tensors.append(x)
-        return _Slot(len(tensors) - 1)
-    if isinstance(x, dict):
-        return {k: _flatten(v, tensors) for k, v in x.items()}
-    if isinstance(x, list):
-        return [_flatten(v, tensors) for v in x]
-    return x
-
-
-def _unflatten(x, tensors):
-    if isinstance(x, _Slot):
-        return tensors[x.i]
-    if isinstance(x, dict):
-        return {k: _unflatten(v, tensors) for k, v in x.items()}
-    if isinstance(x, list):
-        return [_unflatten(v, tensors) for v in x]
-    return x
-
-
-class _Slot:
-    __slots__ = ("i",)
-
-    def __init__(self, i):
-        self.i = i
+# the entries of _Saved that are tensors (params: five more)
+_SAVED_TENSORS = ("q", "k", "v", "b", "w", "mix", "g", "kept", "final")
 
 
 class ChunkNestedGDN2Function(torch.autograd.Function):
@@ -684,17 +760,18 @@ class ChunkNestedGDN2Function(torch.autograd.Function):
         # the working tensors go through save_for_backward, so that activation
         # checkpointing (torch.utils.checkpoint) can drop them after the
         # forward and have them recomputed for the backward
-        tensors = []
-        ctx.skeleton = _flatten(saved, tensors)
-        ctx.save_for_backward(*tensors)
+        if saved is not None:
+            ctx.save_for_backward(*(saved[n] for n in _SAVED_TENSORS), *saved["params"])
+            ctx.saved_config = {n: x for n, x in saved.items()
+                                if n not in _SAVED_TENSORS and n != "params"}
         return o, (final if output_final_state else None)
 
     @staticmethod
     def backward(ctx, do, dfinal):
         L, scale, f, nq, has_init, promotion = ctx.meta
-        sv = _unflatten(ctx.skeleton, ctx.saved_tensors)
-        if sv is None:
-            raise RuntimeError("chunk_nested_gdn2: no saved state for the backward")
+        tensors = ctx.saved_tensors
+        n = len(_SAVED_TENSORS)
+        sv = {**ctx.saved_config, **dict(zip(_SAVED_TENSORS, tensors)), "params": tensors[n:]}
         grads = _backward(sv, do, dfinal, L, scale, f, nq, has_init, promotion)
         (dq, dk, dv, dg, db, dw, dmix, dqb, dkp, dbp, dwp, dgp, dinit) = grads
         dts = ctx.dtypes
@@ -720,13 +797,8 @@ def _cast_grads(grads, dtypes):
              if x is not None and x.dtype == torch.float32 and dt == torch.bfloat16
              and x.is_contiguous()]
     if len(batch) > 1:
-        for i in batch:
-            out[i] = torch.empty(grads[i].shape, device=grads[i].device, dtype=torch.bfloat16)
-        n = len(batch)
-        srcs = (ctypes.c_void_p * n)(*(grads[i].data_ptr() for i in batch))
-        dsts = (ctypes.c_void_p * n)(*(out[i].data_ptr() for i in batch))
-        cnt = (ctypes.c_int64 * n)(*(grads[i].numel() for i in batch))
-        _lib.call("ngdn_cast_bf16", n, srcs, dsts, cnt, _lib.stream_of(grads[batch[0]]))
+        for i, y in zip(batch, _cast_bf16([grads[i] for i in batch])):
+            out[i] = y
     else:
         batch = []
     return [x if x is None or i in batch else x.to(dt)

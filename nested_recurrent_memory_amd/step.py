@@ -35,7 +35,7 @@ def prepare_step_params(query_banks, key_projections, b_projections, w_projectio
                                  b_projections=b_projections, w_projections=w_projections,
                                  g_projections=g_projections)[6:11]
     return _params(query_banks, key_projections, b_projections, w_projections,
-                   g_projections, wd, False)
+                   g_projections, wd)
 
 
 def _validate_step(q, k, v, L, chunk_size, promotion, nq, f, query_banks):
@@ -179,12 +179,20 @@ def step_nested_gdn2(
     fs = (ctypes.c_int32 * L)(*f)
     nqs = (ctypes.c_int32 * max(L - 1, 1))(*(nq or [0]))
     if L > 1:
-        par = params if params is not None else _params(
-            query_banks, key_projections, b_projections, w_projections, g_projections, wd,
-            False)
-        if par["qb"].dtype != wd:
-            raise ValueError(f"params were prepared for {par['qb'].dtype}, inputs are {wd}")
         n_pairs = K if merge else max(nq)
+        if params is not None:
+            par = params
+            if par["qb"].dtype != wd:
+                raise ValueError(f"params were prepared for {par['qb'].dtype}, inputs are {wd}")
+        elif pos_t is None and not any((pos_all + 1) % (int(chunk_size) * x) == 0 for x in f[1:]):
+            # a host position at which no level fires: the parameters are not
+            # read, and are not laid out either (63 of 64 tokens; one sequence,
+            # H = 16, K = 64, two levels: 43 -> 21 us a token)
+            par = dict(qb=query_banks, nmax=-(-query_banks.shape[2] // 8) * 8, kp=key_projections,
+                       bpT=b_projections, wpT=w_projections, gpT=g_projections)
+        else:
+            par = _params(query_banks, key_projections, b_projections, w_projections,
+                          g_projections, wd)
         ws = torch.empty(B * H * (3 * n_pairs * K + K), device=dev, dtype=torch.float32)
     d = _lib.dims(B, 1, H, L, K, V, code, scale)
     _lib.call("ngdn_step", ctypes.byref(d), P(q_), P(k_), P(v_), P(g_), P(b_), P(w_), P(mix_),
