@@ -15,18 +15,25 @@
 
 namespace ngdn {
 
-template <typename E, int K, int V>
+// NL, the number of levels (0: a.L, up to MAXL): known, every load of the
+// thread, all levels' state rows included, is issued before the first use,
+// and an out-of-place step stores the upper rows it holds instead of reading
+// them again. B = 256, H = 16, K = 128, three levels: 219 -> 206 us in place
+// (1.09 GB, 5.3 TB/s: a copy's rate), 332 -> 294 us out of place.
+template <typename E, int K, int V, int NL>
 __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
   constexpr int SV = 32;                 // columns per workgroup
   constexpr int CQ = SV / 4;             // threads across one row (4 columns each)
   constexpr int RG = 256 / CQ;           // row groups
   constexpr int RPT = K / RG;            // rows per thread
   constexpr int NW = 256 / WAVE;
+  constexpr int LM = NL ? NL : MAXL;     // levels the code is laid out for
+  constexpr bool AHEAD = NL > 0;
   static_assert(RPT >= 1 && K % RG == 0, "K must be a multiple of 32");
   __shared__ __attribute__((aligned(16))) float s_red[NW][SV];
-  __shared__ __attribute__((aligned(16))) float s_rd[NW][MAXL][SV];
+  __shared__ __attribute__((aligned(16))) float s_rd[NW][LM][SV];
 
-  const int H = a.H, L = a.L;
+  const int H = a.H, L = NL ? NL : a.L;
   int bh, vs;
   xcd_split(blockIdx.x, gridDim.x, V / SV, bh, vs);
   const int h = bh % H, b = bh / H;
@@ -43,17 +50,41 @@ __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
   float* Sout = a.s_out + sbase;
   const bool copy_up = a.s_out != a.s_in;
 
-  // ---- level 0: decay, erase projection r = (k*b)^T (e^g S0)
-  f4 s0[RPT];
-  float key[RPT];
-  f4 part = f4_zero();
+  // ---- the loads: level 0's rows, the token's rows, the upper levels' rows
+  f4 s0[RPT], up[AHEAD ? LM : 1][RPT];
+  float gl[RPT], key[RPT], bl[RPT];
 #pragma unroll
   for (int r = 0; r < RPT; ++r) {
     const int k = rg * RPT + r;
     s0[r] = *reinterpret_cast<const f4*>(Sin + (size_t)k * V + col);
-    const float gam = expf(gg[k]);
+  }
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int k = rg * RPT + r;
+    gl[r] = gg[k];
     key[r] = to_f(kk[k]);
-    const float kb = key[r] * to_f(bb[k]);
+    bl[r] = to_f(bb[k]);
+  }
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int l = 1; l < LM; ++l)
+#pragma unroll
+      for (int r = 0; r < RPT; ++r)
+        up[l][r] = *reinterpret_cast<const f4*>(Sin + ((size_t)l * K + rg * RPT + r) * V + col);
+  }
+  const E* vv = static_cast<const E*>(a.v) + (size_t)bh * V + col;
+  const E* ww = static_cast<const E*>(a.w) + (size_t)bh * V + col;
+  E v4[4], w4[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) { v4[c] = vv[c]; w4[c] = ww[c]; }
+  if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+
+  // ---- level 0: decay, erase projection r = (k*b)^T (e^g S0)
+  f4 part = f4_zero();
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const float gam = expf(gl[r]);
+    const float kb = key[r] * bl[r];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       s0[r][c] *= gam;
@@ -69,17 +100,17 @@ __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
   if (lane < CQ) *reinterpret_cast<f4*>(&s_red[wv][cq * 4]) = part;
 
   // reads of the upper levels (unchanged by this token)
-  f4 rd[MAXL];
+  f4 rd[LM];
 #pragma unroll
-  for (int l = 0; l < MAXL; ++l) rd[l] = f4_zero();
+  for (int l = 0; l < LM; ++l) rd[l] = f4_zero();
 #pragma unroll
-  for (int l = 1; l < MAXL; ++l) {
+  for (int l = 1; l < LM; ++l) {
     if (l < L) {
       const float* Sl = Sin + (size_t)l * K * V;
 #pragma unroll
       for (int r = 0; r < RPT; ++r) {
         const int k = rg * RPT + r;
-        const f4 x = *reinterpret_cast<const f4*>(Sl + (size_t)k * V + col);
+        const f4 x = AHEAD ? up[AHEAD ? l : 0][r] : *reinterpret_cast<const f4*>(Sl + (size_t)k * V + col);
         const float ql = to_f(q[(size_t)l * K + k]) * a.scale;
 #pragma unroll
         for (int c = 0; c < 4; ++c) rd[l][c] += ql * x[c];
@@ -89,14 +120,12 @@ __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
   lds_barrier();
   f4 u;
   {
-    const E* vv = static_cast<const E*>(a.v) + (size_t)bh * V + col;
-    const E* ww = static_cast<const E*>(a.w) + (size_t)bh * V + col;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       float r = 0.f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) r += s_red[w][cq * 4 + c];
-      u[c] = to_f(vv[c]) * to_f(ww[c]) - r;
+      u[c] = to_f(v4[c]) * to_f(w4[c]) - r;
     }
   }
 
@@ -113,7 +142,7 @@ __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
     for (int c = 0; c < 4; ++c) rd[0][c] += ql * s0[r][c];
   }
 #pragma unroll
-  for (int l = 0; l < MAXL; ++l) {
+  for (int l = 0; l < LM; ++l) {
     if (l < L) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
@@ -123,6 +152,14 @@ __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
       }
       if (lane < CQ) *reinterpret_cast<f4*>(&s_rd[wv][l][cq * 4]) = rd[l];
     }
+  }
+  // out of place: the upper levels are copied last (after every load)
+  if (AHEAD && copy_up) {
+#pragma unroll
+    for (int l = 1; l < LM; ++l)
+#pragma unroll
+      for (int r = 0; r < RPT; ++r)
+        *reinterpret_cast<f4*>(Sout + ((size_t)l * K + rg * RPT + r) * V + col) = up[AHEAD ? l : 0][r];
   }
   lds_barrier();
 
@@ -142,8 +179,7 @@ __global__ __launch_bounds__(256) void step_kernel(StepArgs a) {
       o[c] = from_f<E>(acc);
     }
   }
-  // out of place: the upper levels are copied last (after every load)
-  if (copy_up) {
+  if (!AHEAD && copy_up) {
     for (int l = 1; l < L; ++l) {
 #pragma unroll
       for (int r = 0; r < RPT; ++r) {
@@ -399,36 +435,61 @@ __device__ __forceinline__ void promote_level(const PromoteArgs& a, char* smem, 
   }
 }
 
+// Workgroup x takes the (row, head) pairs x, x + grid, ...: the grid is what
+// the GPU holds at once (the LDS of a promotion leaves one workgroup per CU at
+// K = 128, two at K = 64), and the firing decision of up to 64 of its pairs is
+// made at once, one per lane. With one workgroup per pair, a decoding batch
+// (few of its rows at a chunk's end) passed thousands of workgroups through the
+// CUs one by one only to see them return (B = 256, H = 16, one row firing: 37
+// -> 35 us, the rest being the one promotion's chain of phases). The heads of
+// a firing row go to different workgroups.
 template <typename E, int K>
 __global__ __launch_bounds__(512) void promote_kernel(PromoteArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[PromoteLds<K>::BYTES];
   __shared__ float s_nrm[8 * PROMOTE_NMAX], s_gs[8 * K], s_gam[K];
-  const int bh = blockIdx.x, h = bh % a.H, b = bh / a.H;
-  const long long end = (a.pos ? a.pos[b] : a.pos_all) + 1;
-  if (end % a.chunk != 0) return;
-  const long long nchunk = end / a.chunk;
-  for (int l = 1; l < a.L; ++l) {
-    if (nchunk % a.f[l] != 0) continue;
-    const int N = a.N[l];
-    if (a.merge) {
-      if constexpr (K <= PROMOTE_NMAX) promote_level<E, K, K, true>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
-    } else if (N == 16) {
-      promote_level<E, K, 16, false>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
-    } else if (N == 32) {
-      promote_level<E, K, 32, false>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
-    } else {
-      promote_level<E, K, 64, false>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
+  const long long total = (long long)a.B * a.H, stride = gridDim.x;
+  for (long long i0 = blockIdx.x; i0 < total; i0 += WAVE * stride) {
+    const long long mine = i0 + lane_id() * stride;
+    bool fires = false;
+    if (mine < total) {
+      const long long end = (a.pos ? a.pos[mine / a.H] : a.pos_all) + 1;
+      if (end % a.chunk == 0)
+        for (int l = 1; l < a.L; ++l) fires = fires || (end / a.chunk) % a.f[l] == 0;
     }
-    // the next level's probe reads this level's new state, written by every
-    // wave: a barrier that also orders global memory
-    __syncthreads();
+    // the same in every wave of the workgroup
+    unsigned long long todo = __ballot(fires);
+    while (todo) {
+      const long long bh = i0 + (__ffsll(todo) - 1) * stride;
+      todo &= todo - 1;
+      const int h = (int)(bh % a.H), b = (int)(bh / a.H);
+      const long long nchunk = ((a.pos ? a.pos[b] : a.pos_all) + 1) / a.chunk;
+      for (int l = 1; l < a.L; ++l) {
+        if (nchunk % a.f[l] != 0) continue;
+        const int N = a.N[l];
+        if (a.merge) {
+          if constexpr (K <= PROMOTE_NMAX) promote_level<E, K, K, true>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
+        } else if (N == 16) {
+          promote_level<E, K, 16, false>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
+        } else if (N == 32) {
+          promote_level<E, K, 32, false>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
+        } else {
+          promote_level<E, K, 64, false>(a, smem, s_nrm, s_gs, s_gam, b, h, l);
+        }
+        // the next level's probe reads this level's new state, written by
+        // every wave, and the next level or pair reuses the LDS: a barrier
+        // that also orders global memory
+        __syncthreads();
+      }
+    }
   }
 }
 
 template <typename E, int K>
 static hipError_t launch_promote(const PromoteArgs& a, hipStream_t st) {
-  const unsigned grid = (unsigned)(a.B * a.H);
-  if (grid == 0) return hipSuccess;
+  const long long pairs = (long long)a.B * a.H;
+  if (pairs == 0) return hipSuccess;
+  constexpr long long HELD = K == 128 ? 256 : 512;   // workgroups the CUs hold at once
+  const unsigned grid = (unsigned)(pairs < HELD ? pairs : HELD);
   hipLaunchKernelGGL((promote_kernel<E, K>), dim3(grid), dim3(512), 0, st, a);
   return hipGetLastError();
 }
@@ -446,7 +507,11 @@ hipError_t promote_fwd(const PromoteArgs& a, int dtype, int K, hipStream_t st) {
 template <typename E, int K, int V>
 static hipError_t launch_step(const StepArgs& a, hipStream_t st) {
   const unsigned grid = (unsigned)(a.B * a.H * (V / 32));
-  hipLaunchKernelGGL((step_kernel<E, K, V>), dim3(grid), dim3(256), 0, st, a);
+#define NGDN_SL(NL) \
+  if (a.L == NL) hipLaunchKernelGGL((step_kernel<E, K, V, NL>), dim3(grid), dim3(256), 0, st, a);
+  NGDN_SL(1) NGDN_SL(2) NGDN_SL(3) NGDN_SL(4)
+#undef NGDN_SL
+  if (a.L > 4) hipLaunchKernelGGL((step_kernel<E, K, V, 0>), dim3(grid), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
