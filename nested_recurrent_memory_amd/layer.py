@@ -35,7 +35,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .chunk import chunk_nested_gdn2
-from .layer_ops import FusedRMSNormGated, ShortConvolution, fanout, gate_prep
+from .layer_ops import FusedRMSNormGated, ShortConvolution, first_linear, gate_prep, linears
 from .step import step_nested_gdn2
 
 __all__ = ["NestedGDN2LayerConfig", "NestedGDN2Attention"]
@@ -164,23 +164,29 @@ class NestedGDN2Attention(nn.Module):
         last = past_key_values.get(self.layer_idx) if past_key_values is not None else None
         conv = last.get("conv_state") if last is not None else None
         conv_q, conv_k, conv_v = conv if conv is not None else (None, None, None)
-        # x feeds eight linear maps: one autocast cast of it for all of them
-        xq, xk, xv, xf, xb, xw, xm, xg = fanout(x, 8)
+        # the eight linear maps of x (the first of the two of f and of g)
+        f_in, g_in = first_linear(self.f_proj), first_linear(self.g_proj)
+        q, k, v, f, bz, wz, ml, gz = linears(x, (
+            self.q_proj, self.k_proj, self.v_proj, f_in, self.b_proj, self.w_proj,
+            self.mix_proj, g_in))
+        if f_in is not self.f_proj:
+            f = self.f_proj[1](f)
+        if g_in is not self.g_proj:
+            gz = self.g_proj[1](gz)
         if cfg.use_short_conv:
-            q, conv_q = self.q_conv1d(self.q_proj(xq), cache=conv_q, output_final_state=use_cache)
-            k, conv_k = self.k_conv1d(self.k_proj(xk), cache=conv_k, output_final_state=use_cache)
-            v, conv_v = self.v_conv1d(self.v_proj(xv), cache=conv_v, output_final_state=use_cache)
+            q, conv_q = self.q_conv1d(q, cache=conv_q, output_final_state=use_cache)
+            k, conv_k = self.k_conv1d(k, cache=conv_k, output_final_state=use_cache)
+            v, conv_v = self.v_conv1d(v, cache=conv_v, output_final_state=use_cache)
         else:
-            q, k, v = (F.silu(p(xi)) for p, xi in ((self.q_proj, xq), (self.k_proj, xk),
-                                                    (self.v_proj, xv)))
+            q, k, v = (F.silu(t) for t in (q, k, v))
         v = v.reshape(B, T, H, V)
         # q -> [B,T,H,L,K] and k L2-normalised, the decay g0 (fp32), gates b0,
         # w0 and the level mix, in one kernel (layers/nested_gdn2.py:134-166)
         gated = cfg.read_mix == "sigmoid"
         wd = v.dtype
         q, k, g0, b0, w0, mix = gate_prep(
-            q.to(wd), k.to(wd), self.f_proj(xf).to(wd), self.b_proj(xb).to(wd),
-            self.w_proj(xw).to(wd), self.mix_proj(xm).to(wd), self.A_log, self.dt_bias,
+            q.to(wd), k.to(wd), f.to(wd), bz.to(wd), wz.to(wd), ml.to(wd),
+            self.A_log, self.dt_bias,
             L, H, K, V, max_horizon=cfg.max_horizon, sigmoid_mix=gated)
         keep = getattr(cfg, "read_levels", None)   # eval-time read ablation (not a config field)
         if keep is not None:
@@ -241,5 +247,5 @@ class NestedGDN2Attention(nn.Module):
                 "recurrent_state": (state, position),
                 "conv_state": (conv_q, conv_k, conv_v) if cfg.use_short_conv else None,
             }
-        o = self.o_norm(o, self.g_proj(xg).reshape(B, T, H, V))
+        o = self.o_norm(o, gz.reshape(B, T, H, V))
         return self.o_proj(o.reshape(B, T, H * V)), None, past_key_values
