@@ -69,7 +69,7 @@ const char* ngdn_last_error(void);
  * 0.5.0 took W and U out of ngdn_l0_bwd; 0.6.0 moved the upper levels'
  * lower-state gradients from ngdn_probe_bwd's d_below to an injection that
  * ngdn_upper_scan_bwd adds. */
-#define NGDN_VERSION 1000
+#define NGDN_VERSION 1100
 int32_t ngdn_version(void);
 /* Offload architecture the library was built for ("gfx950"). */
 const char* ngdn_arch(void);
@@ -564,6 +564,12 @@ int32_t ngdn_swiglu_bwd(int32_t dtype, int64_t n, const void* g, const void* u, 
  * consumer. No counterpart in fla; it replaces autograd's accumulation. */
 int32_t ngdn_sum_f32(int32_t dtype, int32_t count, const void* const* xs, int64_t n, float* out,
                      void* stream);
+
+/* out[i] = x[i] s[0] in fp32, rounded to out_dtype; x in x_dtype, both NGDN_F32
+ * or NGDN_BF16 and 16-byte aligned, s one device fp32, any n >= 0. The gradients
+ * the loss keeps from its forward, times the loss's own gradient. */
+int32_t ngdn_scale(int32_t x_dtype, int32_t out_dtype, int64_t n, const void* x, const float* s,
+                   void* out, void* stream);
 
 /* The cross entropy of fla's FusedLinearCrossEntropyLoss
  * (models/modeling_nested_gdn2.py:230-239; mean over the labels that are not

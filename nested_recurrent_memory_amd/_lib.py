@@ -20,7 +20,7 @@ NGDN_BF16 = 1
 # NGDN_VERSION of include/ngdn.h: the interface the signatures below describe.
 # The loader refuses a library of another version (working-tensor layouts and
 # argument meanings changed between versions under unchanged signatures).
-VERSION = 1000
+VERSION = 1100
 
 
 class Dims(ctypes.Structure):
@@ -80,6 +80,7 @@ SIGNATURES = {
     "ngdn_swiglu_fwd": [I32, I64] + [P] * 4,
     "ngdn_swiglu_bwd": [I32, I64] + [P] * 6,
     "ngdn_sum_f32": [I32, I32, P, I64, P, P],
+    "ngdn_scale": [I32, I32, I64, P, P, P, P],
     "ngdn_cross_entropy": [I32, I64, I32, I32, P, P, P, P, I32, P],
 }
 _RESTYPES = {"ngdn_last_error": ctypes.c_char_p, "ngdn_arch": ctypes.c_char_p}

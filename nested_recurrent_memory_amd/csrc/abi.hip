@@ -1065,6 +1065,19 @@ int32_t ngdn_sum_f32(int32_t dtype, int32_t count, const void* const* xs, int64_
   return launched(ngdn::sum_into_f32(a, dtype, (hipStream_t)stream), "ngdn_sum_f32");
 }
 
+int32_t ngdn_scale(int32_t x_dtype, int32_t out_dtype, int64_t n, const void* x, const float* s,
+                   void* out, void* stream) {
+  g_err[0] = 0;
+  for (int32_t d : {x_dtype, out_dtype})
+    if (d != NGDN_F32 && d != NGDN_BF16) return fail(NGDN_EINVAL, "ngdn_scale: dtype %d", d);
+  if (n < 0 || (n > 0 && (!x || !s || !out)))
+    return fail(NGDN_EINVAL, "ngdn_scale: NULL tensor or n=%lld", (long long)n);
+  if (n > 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15))
+    return fail(NGDN_EINVAL, "ngdn_scale: x and out must be 16-byte aligned");
+  ngdn::ScaleArgs a{x, s, out, n};
+  return launched(ngdn::scale(a, x_dtype, out_dtype, (hipStream_t)stream), "ngdn_scale");
+}
+
 int32_t ngdn_cross_entropy(int32_t dtype, int64_t rows, int32_t V, int32_t ignore_index,
                            void* logits, const int64_t* labels, const int64_t* n_valid,
                            float* row_loss, int32_t grad, void* stream) {

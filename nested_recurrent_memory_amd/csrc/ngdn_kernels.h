@@ -306,6 +306,10 @@ struct SumArgs {
 };
 hipError_t sum_into_f32(const SumArgs& a, int dtype, hipStream_t st);
 
+// out[i] = x[i] s[0], n elements (model_ops.hip)
+struct ScaleArgs { const void* x; const float* s; void* out; long long n; };
+hipError_t scale(const ScaleArgs& a, int x_dtype, int out_dtype, hipStream_t st);
+
 // Cross entropy of rows of V logits (model_ops.hip): row_loss[r] =
 // (logsumexp(x_r) - x_r[label_r]) / n_valid, 0 for ignored labels; with grad
 // the logits are overwritten by d(sum of row_loss)/dx = (softmax - onehot) /

@@ -216,6 +216,24 @@ class GatedMLP(nn.Module):
 _BLOCK_BYTES = 4 << 30     # logits held at once
 
 
+def _scaled(x, s, dtype):
+    """x s in fp32, rounded to dtype; s a scalar tensor."""
+    if (x.is_cuda and s.is_cuda and x.device == s.device and s.dtype == torch.float32
+            and x.dtype in _SCALED and dtype in _SCALED and x.is_contiguous()
+            and not torch.is_grad_enabled()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(s)
+            and x.data_ptr() % 16 == 0):
+        out = torch.empty(x.shape, device=x.device, dtype=dtype)
+        _lib.call("ngdn_scale", _code(x), _code(out), x.numel(), _lib.ptr(x), _lib.ptr(s),
+                  _lib.ptr(out), _lib.stream_of(x))
+        return out
+    # differentiated again, or over a batch of gradients
+    return (x.float() * s).to(dtype)
+
+
+_SCALED = (torch.float32, torch.bfloat16)
+
+
 class _LinearCEFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, target, weight, bias, ignore_index):
@@ -234,21 +252,24 @@ class _LinearCEFn(torch.autograd.Function):
         dx = torch.empty_like(xc) if grad else None
         dw = db = None
         rows = max(1, min(N, _BLOCK_BYTES // (V * xc.element_size())))
-        for r0 in range(0, N, rows):
-            r1 = min(N, r0 + rows)
-            logits = xc[r0:r1] @ wc.t()
-            if bc is not None:
-                logits += bc
-            _lib.call("ngdn_cross_entropy", _code(logits), r1 - r0, V, int(ignore_index),
-                      _lib.ptr(logits), _lib.ptr(tgt[r0:r1]), _lib.ptr(n_valid),
-                      _lib.ptr(row_loss[r0:r1]), int(grad), _lib.stream_of(logits))
-            if grad:       # logits now hold d(loss)/d(logits)
-                dx[r0:r1] = logits @ wc
-                part = (logits.t() @ xc[r0:r1]).float()
-                dw = part if dw is None else dw.add_(part)
+        with torch.autocast("cuda", enabled=False):    # everything is in cdt from here
+            for r0 in range(0, N, rows):
+                r1 = min(N, r0 + rows)
+                logits = xc[r0:r1] @ wc.t()
                 if bc is not None:
-                    pb = logits.float().sum(0)
-                    db = pb if db is None else db.add_(pb)
+                    logits += bc
+                _lib.call("ngdn_cross_entropy", _code(logits), r1 - r0, V, int(ignore_index),
+                          _lib.ptr(logits), _lib.ptr(tgt[r0:r1]), _lib.ptr(n_valid),
+                          _lib.ptr(row_loss[r0:r1]), int(grad), _lib.stream_of(logits))
+                if grad:       # logits now hold d(loss)/d(logits)
+                    torch.mm(logits, wc, out=dx[r0:r1])
+                    part = logits.t() @ xc[r0:r1]
+                    if rows < N:       # several blocks: their sum in fp32
+                        part = part.float()
+                    dw = part if dw is None else dw.add_(part)
+                    if bc is not None:
+                        pb = logits.float().sum(0)
+                        db = pb if db is None else db.add_(pb)
         ctx.dtypes = (x.dtype, weight.dtype, bias.dtype if bias is not None else None)
         if grad:
             ctx.save_for_backward(dx, dw, db)
@@ -258,8 +279,8 @@ class _LinearCEFn(torch.autograd.Function):
     def backward(ctx, dloss):
         dx, dw, db = ctx.saved_tensors
         xd, wd, bd = ctx.dtypes
-        gx = (dx * dloss).to(xd) if ctx.needs_input_grad[0] else None
-        gw = (dw * dloss).to(wd) if ctx.needs_input_grad[2] else None
+        gx = _scaled(dx, dloss, xd) if ctx.needs_input_grad[0] else None
+        gw = _scaled(dw, dloss, wd) if ctx.needs_input_grad[2] else None
         gb = (db * dloss).to(bd) if (db is not None and ctx.needs_input_grad[3]) else None
         return gx, None, gw, gb, None
 
