@@ -264,6 +264,16 @@ class _PackFn(torch.autograd.Function):
         return tuple(o if need else None for o, need in zip(out, ctx.needs_input_grad))
 
 
+def _cat_columns(xs):
+    """torch.cat(xs, 1) of bf16 matrices, copied 16 bytes at a time where
+    every row starts at a multiple of 16 bytes (cat copies by element: 8192
+    rows of 7448, 86 -> 39 us)."""
+    if (not torch.is_grad_enabled()
+            and all(x.is_contiguous() and x.shape[1] % 8 == 0 and x.data_ptr() % 16 == 0 for x in xs)):
+        return torch.cat([x.view(torch.complex128) for x in xs], 1).view(xs[0].dtype)
+    return torch.cat(xs, 1)
+
+
 class _LinearsFn(torch.autograd.Function):
     """The rows of w, n_i at a time, applied to one x. Backward: the output
     gradients side by side, so that dx and dw are one GEMM each, and dx one
@@ -286,8 +296,8 @@ class _LinearsFn(torch.autograd.Function):
         rows = x2.shape[0]
         dx = dw = None
         with torch.autocast("cuda", enabled=False):
-            dy = torch.cat([g.reshape(rows, n) if g is not None else x2.new_zeros(rows, n)
-                            for g, n in zip(grads, ctx.ns)], dim=1)
+            dy = _cat_columns([g.reshape(rows, n) if g is not None else x2.new_zeros(rows, n)
+                               for g, n in zip(grads, ctx.ns)])
             if ctx.needs_input_grad[0]:
                 dx = torch.mm(dy, w).view(x.shape)
             if ctx.needs_input_grad[1]:

@@ -24,9 +24,10 @@ def _mods(d, widths, dtype):
 
 
 @pytest.mark.parametrize("rows", [(1, 1), (2, 37), (3, 128)])
+@pytest.mark.parametrize("widths", [(128, 24, 3, 64), (128, 24, 8, 64)])   # columns in 16 bytes or not
 @pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
-def test_linears_match_the_modules(rows, wdtype):
-    d, widths = 64, (128, 24, 3, 64)
+def test_linears_match_the_modules(rows, widths, wdtype):
+    d = 64
     mods = _mods(d, widths, wdtype)
     mods[1].weight.requires_grad_(False)
     x = torch.randn(*rows, d, device="cuda").bfloat16().requires_grad_(True)
