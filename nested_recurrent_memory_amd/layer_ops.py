@@ -325,13 +325,15 @@ def first_linear(seq):
 
 def linears(x, mods):
     """[m(x) for m in mods] for linear maps of one x: through _LinearsFn where
-    gradients are recorded, x is bf16 on the GPU and the maps are plain
-    bias-free nn.Linear with contiguous weights of one dtype, bf16 or, under
-    bf16 autocast, fp32; the modules themselves otherwise (with one autocast
-    cast of x, see fanout): without a backward there is nothing to join, and
-    autocast may hold a weight's cast from one call for the next."""
+    gradients are recorded, x is bf16 on the GPU, of 64 rows or more, and the
+    maps are plain bias-free nn.Linear with contiguous weights of one dtype,
+    bf16 or, under bf16 autocast, fp32; the modules themselves otherwise (with
+    one autocast cast of x, see fanout). Without a backward there is nothing
+    to join, and autocast may hold a weight's cast from one call for the next,
+    which a decoding loop's few rows live from, also where gradients are on."""
     ws = [getattr(m, "weight", None) for m in mods]
-    if (x.dtype == torch.bfloat16 and x.is_cuda and x.numel() and torch.is_grad_enabled()
+    if (x.dtype == torch.bfloat16 and x.is_cuda and torch.is_grad_enabled()
+            and x.numel() >= 64 * x.shape[-1] > 0
             and x.get_device() == torch.cuda.current_device() and len(mods) <= 16
             and all(_plain_linear(m) for m in mods) and not _global_hooks()
             and all(w.dtype == ws[0].dtype and w.device == x.device and w.is_contiguous()

@@ -2,7 +2,7 @@
 themselves: bf16 x with fp32 weights under bf16 autocast and with bf16
 weights, odd widths, weights that want no gradient, outputs that go unused;
 and the forms that must go through the modules (hooks, fp32 x, a bias, a
-subclass). Bounds: outputs are the same products; gradients are sums of bf16
+subclass, no gradients, few rows). Bounds: outputs are the same products; gradients are sums of bf16
 values rounded once instead of once per map."""
 
 import pytest
@@ -23,7 +23,7 @@ def _mods(d, widths, dtype):
     return [nn.Linear(d, n, bias=False).cuda().to(dtype) for n in widths]
 
 
-@pytest.mark.parametrize("rows", [(1, 1), (2, 37), (3, 128)])
+@pytest.mark.parametrize("rows", [(1, 64), (2, 37), (3, 128)])
 @pytest.mark.parametrize("widths", [(128, 24, 3, 64), (128, 24, 8, 64)])   # columns in 16 bytes or not
 @pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
 def test_linears_match_the_modules(rows, widths, wdtype):
@@ -60,12 +60,12 @@ class _Sub(nn.Linear):
 
 
 @pytest.mark.parametrize("case", ["hook", "fp32 x", "bias", "subclass", "no autocast",
-                                  "fp16 autocast", "no grad"])
+                                  "fp16 autocast", "no grad", "few rows"])
 def test_other_forms_go_through_the_modules(case, monkeypatch):
     monkeypatch.setattr(_LinearsFn, "apply", lambda *a: pytest.fail("fused"))
     mods = _mods(64, (64, 32), torch.bfloat16 if case == "fp16 autocast" else torch.float32)
     seen = []
-    x = torch.randn(4, 64, device="cuda").bfloat16()
+    x = torch.randn(63 if case == "few rows" else 64, 64, device="cuda").bfloat16()
     if case == "hook":
         mods[0].register_forward_hook(lambda m, a, y: seen.append(y.shape))
     elif case == "fp32 x":
@@ -87,7 +87,7 @@ def test_other_forms_go_through_the_modules(case, monkeypatch):
 
 def test_second_derivatives_are_the_modules():
     mods = _mods(32, (8, 24), torch.bfloat16)
-    x = torch.randn(5, 32, device="cuda").bfloat16().requires_grad_(True)
+    x = torch.randn(65, 32, device="cuda").bfloat16().requires_grad_(True)
     ws = [m.weight for m in mods]
 
     def second(ys):
