@@ -288,7 +288,13 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
 
       // ---- Vn = U - A S (and, OUT, the read's Qg S on the same tiles)
       constexpr int CTV = ONE_RT ? NVP : CT;     // column tiles this wave's Vn tiles use
-      auto vn_ct = [&](int c) { return ONE_RT ? (wv + NWV * c) / RTV : c; };
+      // (16 pairs, or 32 in 16 columns, leave some waves without a Vn tile: the
+      // read, kept unconditional, then takes the last column tile, unused)
+      auto vn_ct = [&](int c) {
+        if (!ONE_RT) return c;
+        const int ct = (wv + NWV * c) / RTV;
+        return NVT % NWV == 0 ? ct : min(ct, CT - 1);
+      };
       f4 rd[OUT ? NVP : 1];
       {
         SF fb[CTV][NSK];

@@ -35,13 +35,33 @@ def lanes():
 
 
 class SplitLDS:
-    """A split bf16 tile: hi plane, then lo plane, ``plane`` elements apart."""
+    """A split bf16 tile: hi plane, then lo plane, ``plane`` elements apart;
+    one plane of fp32 values with ``planes=1``."""
 
-    def __init__(self, name, plane):
-        self.name, self.plane = name, plane
+    def __init__(self, name, plane, planes=2):
+        self.name, self.plane, self.planes = name, plane, planes
 
     def span(self, off, n):
-        return [(self.name, p * self.plane + off + e) for p in (0, 1) for e in range(n)]
+        return [(self.name, p * self.plane + off + e) for p in range(self.planes)
+                for e in range(n)]
+
+    @property
+    def size(self):
+        return self.planes * self.plane
+
+
+class Form:
+    """An operand type's matrix-core shape and LDS row padding
+    (csrc/ngdn_common.h Mma, SplitTile), in elements."""
+
+    def __init__(self, KS, KPL, PAD, planes, bytes):
+        self.KS, self.KPL, self.PAD, self.planes, self.bytes = KS, KPL, PAD, planes, bytes
+
+    def kofs(self, l):
+        return self.KPL * (l >> 4)
+
+
+FORMS = {"bf16": Form(32, 8, 8, 2, 2), "fp32": Form(16, 4, 4, 1, 4)}
 
 
 class Phase:
@@ -92,23 +112,31 @@ def acc_row(l, r=0):
 
 # --------------------------------------------------------------- forward scan
 
-def scan_fwd_step(K, M, OUT, NWV=4):
-    """csrc/scan.hip scan_fwd_kernel, bf16 (KS = 32, KPL = 8, PAD = 8)."""
-    KS, PAD = 32, 8
-    LDS_ST, LDS_VN = K + PAD, M + PAD
-    sST, sVn = SplitLDS("st", BV * LDS_ST), SplitLDS("vn", BV * LDS_VN)
+def scan_fwd_step(dtype, K, M, BV, OUT, NWV=4):
+    """csrc/scan.hip scan_fwd_kernel."""
+    F = FORMS[dtype]
+    CT = BV // 16
+    LDS_ST, LDS_VN = K + F.PAD, M + F.PAD
+    sST = SplitLDS("st", BV * LDS_ST, F.planes)
+    sVn = SplitLDS("vn", BV * LDS_VN, F.planes)
     RTS, RTV = K // 16, M // 16
     TPW = RTS * CT // NWV
     NVT = RTV * CT
     NVP = -(-NVT // NWV)
     ONE_RT = NWV % RTV == 0
-    NSK, NSM = K // KS, -(-M // KS)
+    NSK, NSM = K // F.KS, -(-M // F.KS)
+    assert TPW >= 1 and (ONE_RT or RTV % NWV == 0) and (not OUT or (ONE_RT and RTV == NWV))
 
     def vn_tile(wv, p):
         if ONE_RT:
             g = wv + NWV * p
             return g < NVT, g % RTV, g // RTV
         return True, wv + NWV * (p // CT), p % CT
+
+    # the column tile of a wave's c-th set of state fragments: read by every
+    # wave, also by one that has no Vn tile of that number
+    def vn_ct(wv, c):
+        return min((wv + NWV * c) // RTV, CT - 1) if ONE_RT else c
 
     A, B, C = Phase(), Phase(), Phase()
     for wv in range(NWV):
@@ -117,34 +145,31 @@ def scan_fwd_step(K, M, OUT, NWV=4):
                 g = wv * TPW + i
                 rt, ct = g // CT, g % CT
                 A.write(wv, sST.span((ct * 16 + (l & 15)) * LDS_ST + rt * 16 + acc_row(l), 4))
+            for c in range(NVP if ONE_RT else CT):
+                brow = (vn_ct(wv, c) * 16 + (l & 15)) * LDS_ST + F.kofs(l)
+                for s in range(NSK):
+                    B.read(wv, sST.span(brow + s * F.KS, F.KPL))
             for p in range(NVP):
                 ok, rt, ct = vn_tile(wv, p)
-                if not ok:
-                    continue
-                brow = (ct * 16 + (l & 15)) * LDS_ST + 8 * (l >> 4)
-                for s in range(NSK):
-                    B.read(wv, sST.span(brow + s * KS, 8))
-                B.write(wv, sVn.span((ct * 16 + (l & 15)) * LDS_VN + rt * 16 + acc_row(l), 4))
-                if OUT:
-                    vrow = (ct * 16 + (l & 15)) * LDS_VN + 8 * (l >> 4)
-                    for s in range(NSM):
-                        C.read(wv, sVn.span(vrow + s * KS, 8))
-            for i in range(TPW):
-                ct = (wv * TPW + i) % CT
-                vrow = (ct * 16 + (l & 15)) * LDS_VN + 8 * (l >> 4)
+                if ok:     # the products use the set read for the tile's column
+                    assert vn_ct(wv, p if ONE_RT else p % CT) == ct
+                    B.write(wv, sVn.span((ct * 16 + (l & 15)) * LDS_VN + rt * 16 + acc_row(l), 4))
+            for ct in range(CT):
+                vrow = (ct * 16 + (l & 15)) * LDS_VN + F.kofs(l)
                 for s in range(NSM):
-                    if s * KS + 8 * (l >> 4) < M:
-                        C.read(wv, sVn.span(vrow + s * KS, 8))
-    bounds = {"st": 2 * BV * LDS_ST, "vn": 2 * BV * LDS_VN}
+                    if s * F.KS + F.kofs(l) < M:
+                        C.read(wv, sVn.span(vrow + s * F.KS, F.KPL))
     # no barrier at the end of a step: C runs together with the next step's A
-    return [A, B, merged(C, A)], bounds
+    return [A, B, merged(C, A)], {"st": sST.size, "vn": sVn.size}
 
 
-@pytest.mark.parametrize("K,M,OUT", [(128, 64, True), (64, 64, True), (128, 64, False),
-                                     (128, 32, False), (128, 16, False), (128, 128, False),
-                                     (64, 128, False)])
-def test_forward_scan_phases(K, M, OUT):
-    phases, bounds = scan_fwd_step(K, M, OUT)
+@pytest.mark.parametrize("M,OUT", [(64, True), (16, False), (32, False), (64, False),
+                                   (128, False)])
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("BV", [16, 32])
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+def test_forward_scan_phases(dtype, BV, K, M, OUT):
+    phases, bounds = scan_fwd_step(dtype, K, M, BV, OUT)
     check_phases(phases, bounds)
 
 
