@@ -450,9 +450,9 @@ __device__ __forceinline__ void stage_split(const ST& dst, int ld, const float* 
 
 // At the end of a loop body (or ahead of a branch) whose last products are
 // read on the other side: an MFMA's result may be read only a number of wait
-// states after it (8 for the 16x16x32 bf16, 10 for the 16x16x4 fp32), which
-// the compiler keeps within a block but was seen to leave short across a
-// branch (too few states: the last rows of a tile came out stale).
+// states after it (8 for the 16x16x32 bf16, 10 for the 16x16x4 fp32). One
+// build of an unrolled forward scan had too few of them across its loop's
+// branch, and the last rows of a tile came out stale; here they are written.
 __device__ __forceinline__ void mfma_settle() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_nop 11");

@@ -351,6 +351,7 @@ __global__ __launch_bounds__(NWV * WAVE) void scan_fwd_kernel(ScanArgs a) {
           for (int s = 0; s < NSM; ++s) rd[p] = Mma<E>::mma(rd[p], cur.aq[0][s], fv[p][s]);
           prd[p] = rd[p];
         }
+        if constexpr (SM == 0) mfma_settle();   // its stores stand under branches
       }
       load(P3{}, jn, nxt);
       // ---- this step's stores (the state registers still hold the state
