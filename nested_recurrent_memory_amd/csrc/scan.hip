@@ -455,7 +455,7 @@ static hipError_t launch_scan_frm(const ScanArgs& a, int sm, hipStream_t st) {
   if constexpr (M == CH && FRM != 1) {
     if (sm == 1) return launch_scan_sm<E, K, M, BV, true, FRM, 1>(a, st);
     if (sm == 2) return launch_scan_sm<E, K, M, BV, true, FRM, 2>(a, st);
-    if constexpr (BV == SCAN_BV) {
+    if constexpr (BV == SCAN_BV || FRM) {
       if (a.read0) return launch_scan_sm<E, K, M, BV, true, FRM, 0>(a, st);
     }
   }
@@ -463,7 +463,7 @@ static hipError_t launch_scan_frm(const ScanArgs& a, int sm, hipStream_t st) {
   if constexpr (FRM != 3) {
     if (sm == 3) return launch_scan_sm<E, K, M, BV, false, FRM, 3>(a, st);
   }
-  if constexpr (BV == SCAN_BV) return launch_scan_sm<E, K, M, BV, false, FRM, 0>(a, st);
+  if constexpr (BV == SCAN_BV || FRM) return launch_scan_sm<E, K, M, BV, false, FRM, 0>(a, st);
   return hipErrorInvalidValue;
 }
 
@@ -485,9 +485,12 @@ static hipError_t launch_scan(const ScanArgs& a, hipStream_t st) {
   // Few (batch, head) pairs (a long sequence in a small batch): 16-column
   // slices, twice the workgroups with half the products per step each; a
   // step's operands are then read by twice as many workgroups, which costs
-  // more than it saves once the grid fills the chip.
+  // more than it saves once the grid fills the chip. The general outputs have
+  // the narrow form where the operands are in fragment order: a decoded token
+  // whose level takes 128 pairs, K = 128, one sequence of 16 heads, 47.7 -> 46.3
+  // us (merge 34.0 -> 32.5).
   const int sm = scan_outputs(a);
-  if (sm && a.B * a.H * (a.V / SCAN_BV) <= SCAN_NARROW_GRID)
+  if ((sm || a.frag) && a.B * a.H * (a.V / SCAN_BV) <= SCAN_NARROW_GRID)
     return launch_scan_bv<E, K, M, 16>(a, sm, st);
   return launch_scan_bv<E, K, M, SCAN_BV>(a, sm, st);
 }
