@@ -2,13 +2,14 @@
 
 The forward and reverse scans pass tiles between the waves of a workgroup
 through LDS: the state (or its gradient) transposed, Vn (or dVn), and in the
-level-0 reverse scan mix_0 dO and every wave's private copy of its operand
-slices. A workgroup barrier separates the phases of a step; where a step
-ends without one, its last phase runs together with the next step's first.
-For every kernel configuration the op launches, this test enumerates, per
-phase, the LDS elements each wave writes and reads (both planes of a split
-tile), from the same index formulas as the kernels (csrc/scan.hip,
-csrc/scan_bwd.hip), and checks:
+level-0 reverse scan mix_0 dO, in two buffers taken in turn, and every wave's
+private copy of its operand slices. A workgroup barrier separates the phases
+of a step; no step ends with one, so its last phase runs together with the
+next step's first. For every kernel configuration the op launches (both types,
+slices of 16 and 32 columns), this test enumerates, per phase, the LDS
+elements each wave writes and reads (both planes of a split tile), from the
+same index formulas as the kernels (csrc/scan.hip, csrc/scan_bwd.hip), and
+checks:
 
   * no element is written by one wave and read or written by another within
     one phase (including the merged end-of-step / start-of-step phase);
@@ -26,8 +27,6 @@ import itertools
 import pytest
 
 WAVE = 64
-BV = 32          # columns of V per scan workgroup
-CT = BV // 16
 
 
 def lanes():
@@ -175,15 +174,17 @@ def test_forward_scan_phases(dtype, BV, K, M, OUT):
 
 # ------------------------------------------------------- reverse scan, levels >= 1
 
-def scan_bwd_upper_step(K, M):
-    """csrc/scan_bwd.hip scan_bwd_kernel, bf16: dS'^T then dVn^T; no barrier
-    at the end of a step."""
-    KS, PAD = 32, 8
-    LDS_ST, LDS_VN = K + PAD, M + PAD
-    sdS, sdV = SplitLDS("dst", BV * LDS_ST), SplitLDS("dvn", BV * LDS_VN)
+def scan_bwd_upper_step(dtype, K, M, BV):
+    """csrc/scan_bwd.hip scan_bwd_kernel: dS'^T then dVn^T; no barrier at the
+    end of a step."""
+    F = FORMS[dtype]
+    CT = BV // 16
+    LDS_ST, LDS_VN = K + F.PAD, M + F.PAD
+    sdS = SplitLDS("dst", BV * LDS_ST, F.planes)
+    sdV = SplitLDS("dvn", BV * LDS_VN, F.planes)
     RTS, RTV = K // 16, M // 16
     TPW, RPW = RTS * CT // 4, -(-RTV // 4)
-    NSK, NSM = K // KS, -(-M // KS)
+    NSK, NSM = K // F.KS, -(-M // F.KS)
     A, B, C = Phase(), Phase(), Phase()
     for wv in range(4):
         for l in lanes():
@@ -196,24 +197,25 @@ def scan_bwd_upper_step(K, M):
                 if rt >= RTV:
                     continue
                 for ct in range(CT):
-                    srow = (ct * 16 + (l & 15)) * LDS_ST + 8 * (l >> 4)
+                    srow = (ct * 16 + (l & 15)) * LDS_ST + F.kofs(l)
                     for s in range(NSK):
-                        B.read(wv, sdS.span(srow + s * KS, 8))
+                        B.read(wv, sdS.span(srow + s * F.KS, F.KPL))
                     B.write(wv, sdV.span((ct * 16 + (l & 15)) * LDS_VN + rt * 16 + acc_row(l), 4))
             for i in range(TPW):
                 ct = i % CT
-                vrow = (ct * 16 + (l & 15)) * LDS_VN + 8 * (l >> 4)
+                vrow = (ct * 16 + (l & 15)) * LDS_VN + F.kofs(l)
                 for s in range(NSM):
-                    if s * KS + 8 * (l >> 4) < M:
-                        C.read(wv, sdV.span(vrow + s * KS, 8))
-    bounds = {"dst": 2 * BV * LDS_ST, "dvn": 2 * BV * LDS_VN}
-    return [A, B, merged(C, A)], bounds
+                    if s * F.KS + F.kofs(l) < M:
+                        C.read(wv, sdV.span(vrow + s * F.KS, F.KPL))
+    return [A, B, merged(C, A)], {"dst": sdS.size, "dvn": sdV.size}
 
 
-@pytest.mark.parametrize("K,M", [(128, 64), (128, 128), (128, 32), (128, 16), (64, 64),
-                                 (64, 16)])
-def test_reverse_scan_upper_phases(K, M):
-    phases, bounds = scan_bwd_upper_step(K, M)
+@pytest.mark.parametrize("M", [16, 32, 64, 128])
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("BV", [16, 32])
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+def test_reverse_scan_upper_phases(dtype, BV, K, M):
+    phases, bounds = scan_bwd_upper_step(dtype, K, M, BV)
     check_phases(phases, bounds)
 
 
@@ -309,23 +311,31 @@ def test_transposed_reads_are_bank_conflict_free():
                         assert len(banks) == 64, (ncw, R, ctl, s, hh, half)
 
 
-def scan_bwd_l0_step(K):
-    """csrc/scan_bwd.hip scan_bwd_l0_kernel, bf16 (M = 64): slice copies,
-    dS'^T and (mix_0 dO)^T, then dVn^T; a barrier ends the step."""
-    M, KS, PAD = 64, 32, 8
-    LDS_ST, LDS_VN = K + PAD, M + PAD
-    sdS, sdV, sdO = (SplitLDS("dst", BV * LDS_ST), SplitLDS("dvn", BV * LDS_VN),
-                     SplitLDS("dot", BV * LDS_VN))
+def scan_bwd_l0_step(dtype, K, BV, which):
+    """csrc/scan_bwd.hip scan_bwd_l0_kernel (M = 64), one step: dS'^T and
+    (mix_0 dO)^T, the latter into buffer ``which``; then dVn^T; then the state
+    gradient. bf16: every wave copies its operand slices first, those of the
+    last products (W, Qg) only beside the dVn products where the halves are
+    placed apart. Two barriers, none at the end. Returns the phases, the
+    buffers' sizes and the elements of a wave's copies."""
+    F = FORMS[dtype]
+    CT = BV // 16
+    M, KS = 64, F.KS
+    LDS_ST, LDS_VN = K + F.PAD, M + F.PAD
+    sdS, sdV, sdO = (SplitLDS(n, BV * ld, F.planes) for n, ld in (
+        ("dst", LDS_ST), ("dvn", LDS_VN), (f"dot{which}", LDS_VN)))
     TPW = (K // 16) * CT // 4
     TRT = TPW // CT
     ncw = 16 * TRT
     DOE = M * BV // 256
+    apart = K < 128 or BV < 32
+    slices = dtype == "bf16"
 
     def plane(R, n):
         return (R // 16) * (16 * n // 8) * 8
 
     pk, pq, pw = plane(K, 16), plane(M, 16), plane(M, ncw)
-    opw = 2 * (pk + pq + 2 * pw)
+    opw = 2 * (pk + pq + 2 * pw) if slices else 0
     regions = {"K": (0, pk, K, 16), "Q": (2 * pk, pq, M, 16), "W": (2 * (pk + pq), pw, M, ncw),
                "G": (2 * (pk + pq) + 2 * pw, pw, M, ncw)}
 
@@ -333,14 +343,22 @@ def scan_bwd_l0_step(K):
         base, pl, _, _ = regions[reg]
         return [("op", wv * opw + base + p * pl + o) for p in (0, 1) for o in offs]
 
+    def read_slice(ph, wv, l, reg, ctl, steps):
+        if slices:
+            for s in range(steps):
+                for hh in range(2):
+                    a = tr_addr(regions[reg][3], l, ctl, s, hh)
+                    ph.read(wv, op_cells(wv, reg, range(a, a + 4)))
+
     A, B, C = Phase(), Phase(), Phase()
     for wv in range(4):
-        for reg, (base, pl, R, n) in regions.items():
+        for reg, (_, _, R, n) in regions.items() if slices else ():
+            ph = B if apart and reg in "WG" else A
             for i in range(R * n // 512):
                 for l in lanes():
                     rb, r, cq = seg_of(n, i, l)
                     d = (rb * (16 * n // 8) + slice_pos(n, r, cq)) * 8
-                    A.write(wv, op_cells(wv, reg, range(d, d + 8)))
+                    ph.write(wv, op_cells(wv, reg, range(d, d + 8)))
         for l in lanes():
             tid = wv * WAVE + l
             for i in range(TPW):
@@ -350,48 +368,51 @@ def scan_bwd_l0_step(K):
             c, vl = tid // (BV // DOE), (tid % (BV // DOE)) * DOE
             for q in range(DOE):
                 A.write(wv, sdO.span((vl + q) * LDS_VN + c, 1))
-            for s in range(K // KS):
-                for hh in range(2):
-                    a = tr_addr(16, l, 0, s, hh)
-                    B.read(wv, op_cells(wv, "K", range(a, a + 4)))
-            for s in range(M // KS):
-                for hh in range(2):
-                    a = tr_addr(16, l, 0, s, hh)
-                    B.read(wv, op_cells(wv, "Q", range(a, a + 4)))
+            read_slice(B, wv, l, "K", 0, K // KS)
+            read_slice(B, wv, l, "Q", 0, M // KS)
             for ct in range(CT):
-                srow = (ct * 16 + (l & 15)) * LDS_ST + 8 * (l >> 4)
-                orow = (ct * 16 + (l & 15)) * LDS_VN + 8 * (l >> 4)
+                srow = (ct * 16 + (l & 15)) * LDS_ST + F.kofs(l)
+                orow = (ct * 16 + (l & 15)) * LDS_VN + F.kofs(l)
                 for s in range(K // KS):
-                    B.read(wv, sdS.span(srow + s * KS, 8))
+                    B.read(wv, sdS.span(srow + s * KS, F.KPL))
                 for s in range(M // KS):
-                    B.read(wv, sdO.span(orow + s * KS, 8))
+                    B.read(wv, sdO.span(orow + s * KS, F.KPL))
                 B.write(wv, sdV.span((ct * 16 + (l & 15)) * LDS_VN + wv * 16 + acc_row(l), 4))
             for t in range(TRT):
-                for s in range(M // KS):
-                    for hh in range(2):
-                        a = tr_addr(ncw, l, t, s, hh)
-                        C.read(wv, op_cells(wv, "W", range(a, a + 4)))
-                        C.read(wv, op_cells(wv, "G", range(a, a + 4)))
+                read_slice(C, wv, l, "W", t, M // KS)
+                read_slice(C, wv, l, "G", t, M // KS)
                 for ct in range(CT):
-                    vrow = (ct * 16 + (l & 15)) * LDS_VN + 8 * (l >> 4)
+                    vrow = (ct * 16 + (l & 15)) * LDS_VN + F.kofs(l)
                     for s in range(M // KS):
-                        C.read(wv, sdV.span(vrow + s * KS, 8))
-                        C.read(wv, sdO.span(vrow + s * KS, 8))
-    bounds = {"dst": 2 * BV * LDS_ST, "dvn": 2 * BV * LDS_VN, "dot": 2 * BV * LDS_VN,
-              "op": 4 * opw}
+                        C.read(wv, sdV.span(vrow + s * KS, F.KPL))
+                        C.read(wv, sdO.span(vrow + s * KS, F.KPL))
+    bounds = {"dst": sdS.size, "dvn": sdV.size, "dot0": sdO.size, "dot1": sdO.size, "op": 4 * opw}
     # each wave touches only its own region of the slice copies
     for ph in (A, B, C):
         for wv, cells in list(ph.w.items()) + list(ph.r.items()):
             for name, e in cells:
                 if name == "op":
                     assert wv * opw <= e < (wv + 1) * opw, (wv, e)
-    # the step ends with a barrier
-    return [A, B, C], bounds, opw
+    return [A, B, C], bounds
 
 
-@pytest.mark.parametrize("K", [128, 64])
-def test_reverse_scan_level0_phases(K):
-    phases, bounds, opw = scan_bwd_l0_step(K)
-    check_phases(phases, bounds)
+def two_steps(even, odd):
+    """The phases of a step and the next, and the start of the one after:
+    what no barrier separates runs together."""
+    return [even[0], even[1], merged(even[2], odd[0]), odd[1], merged(odd[2], even[0])]
+
+
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("BV", [16, 32])
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+def test_reverse_scan_level0_phases(dtype, BV, K):
+    even, bounds = scan_bwd_l0_step(dtype, K, BV, 0)
+    odd, _ = scan_bwd_l0_step(dtype, K, BV, 1)
+    for step in (even, odd):
+        check_phases(step, bounds)       # a step reads what it has written itself
+    check_phases(two_steps(even, odd), bounds)
+    # with one buffer for dO the steps would need a barrier between them
+    with pytest.raises(AssertionError, match="reads what wave"):
+        check_phases(two_steps(even, even), bounds)
     # the whole LDS of the kernel fits one CU (160 KB)
-    assert (bounds["dst"] + bounds["dvn"] + bounds["dot"] + bounds["op"]) * 2 <= 160 * 1024
+    assert sum(bounds.values()) * FORMS[dtype].bytes <= 160 * 1024
