@@ -310,17 +310,28 @@ def _no_hooks(m):
                 or m._backward_pre_hooks)
 
 
+# the forwards that linears() and first_linear() stand in for
+_FORWARD = {c: c.forward for c in (nn.Linear, nn.Sequential)}
+
+
+def _own_forward(m, cls):
+    """m is a cls (no subclass) that runs torch's forward: none set on the
+    instance or in the class's place."""
+    return type(m) is cls and "forward" not in m.__dict__ and cls.forward is _FORWARD[cls]
+
+
 def _plain_linear(m):
     """An nn.Linear without a bias that a call would run as it is: no
-    subclass or parametrization, no hooks, its weight an ordinary parameter."""
-    return (type(m) is nn.Linear and type(m.weight) is nn.Parameter and m.bias is None
+    subclass, patch or parametrization, no hooks, its weight an ordinary
+    parameter."""
+    return (_own_forward(m, nn.Linear) and type(m.weight) is nn.Parameter and m.bias is None
             and _no_hooks(m))
 
 
 def first_linear(seq):
     """The first of a plain two-module nn.Sequential (no hooks), whose caller
     then applies the second; any other module as it is."""
-    return seq[0] if type(seq) is nn.Sequential and len(seq) == 2 and _no_hooks(seq) else seq
+    return seq[0] if _own_forward(seq, nn.Sequential) and len(seq) == 2 and _no_hooks(seq) else seq
 
 
 def linears(x, mods):

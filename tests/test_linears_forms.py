@@ -1,0 +1,29 @@
+"""Which maps the layer may join (linears) and which must run as modules."""
+
+import types
+
+import pytest
+import torch
+import torch.nn as nn
+
+from nested_recurrent_memory_amd import layer_ops
+from nested_recurrent_memory_amd.layer_ops import _plain_linear, first_linear
+
+
+def _linear():
+    return nn.Linear(8, 8, bias=False)
+
+
+def test_a_patched_forward_runs_as_a_module(monkeypatch):
+    """A forward set on an instance, as wrappers that patch modules in place
+    set it, or on the class."""
+    m, seq = _linear(), nn.Sequential(_linear(), _linear())
+    assert _plain_linear(m) and first_linear(seq) is seq[0]
+    m.forward = types.MethodType(lambda self, x: x, m)
+    assert not _plain_linear(m)
+    seq.forward = types.MethodType(lambda self, x: x, seq)
+    assert first_linear(seq) is seq
+    m, seq = _linear(), nn.Sequential(_linear(), _linear())
+    monkeypatch.setattr(nn.Linear, "forward", lambda self, x: x)
+    monkeypatch.setattr(nn.Sequential, "forward", lambda self, x: x)
+    assert not _plain_linear(m) and first_linear(seq) is seq
