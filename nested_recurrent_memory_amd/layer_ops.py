@@ -329,9 +329,10 @@ def _plain_linear(m):
 
 
 def first_linear(seq):
-    """The first of a plain two-module nn.Sequential (no hooks), whose caller
-    then applies the second; any other module as it is."""
-    return seq[0] if _own_forward(seq, nn.Sequential) and len(seq) == 2 and _no_hooks(seq) else seq
+    """The first of a plain two-module nn.Sequential (no hooks, its own or
+    global), whose caller then applies the second; any other module as it is."""
+    return (seq[0] if _own_forward(seq, nn.Sequential) and len(seq) == 2 and _no_hooks(seq)
+            and not _global_hooks() else seq)
 
 
 def linears(x, mods):

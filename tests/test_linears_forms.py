@@ -6,7 +6,6 @@ import pytest
 import torch
 import torch.nn as nn
 
-from nested_recurrent_memory_amd import layer_ops
 from nested_recurrent_memory_amd.layer_ops import _plain_linear, first_linear
 
 
@@ -27,3 +26,15 @@ def test_a_patched_forward_runs_as_a_module(monkeypatch):
     monkeypatch.setattr(nn.Linear, "forward", lambda self, x: x)
     monkeypatch.setattr(nn.Sequential, "forward", lambda self, x: x)
     assert not _plain_linear(m) and first_linear(seq) is seq
+
+
+@pytest.mark.parametrize("register", ["register_module_forward_hook", "register_module_forward_pre_hook",
+                                      "register_module_full_backward_hook"])
+def test_a_global_hook_sees_the_sequential(register):
+    seq = nn.Sequential(_linear(), _linear())
+    handle = getattr(nn.modules.module, register)(lambda *a: None)
+    try:
+        assert first_linear(seq) is seq
+    finally:
+        handle.remove()
+    assert first_linear(seq) is seq[0]
