@@ -337,12 +337,13 @@ def first_linear(seq):
 
 def linears(x, mods):
     """[m(x) for m in mods] for linear maps of one x: through _LinearsFn where
-    gradients are recorded, x is bf16 on the GPU, of 64 rows or more, and the
-    maps are plain bias-free nn.Linear with contiguous weights of one dtype,
-    bf16 or, under bf16 autocast, fp32; the modules themselves otherwise (with
-    one autocast cast of x, see fanout). Without a backward there is nothing
-    to join, and autocast may hold a weight's cast from one call for the next,
-    which a decoding loop's few rows live from, also where gradients are on."""
+    gradients are on and x or a weight wants one, x is bf16 on the GPU, of 64
+    rows or more, and the maps are plain bias-free nn.Linear with contiguous
+    weights of one dtype, bf16 or, under bf16 autocast, fp32; the modules
+    themselves otherwise (with one autocast cast of x, see fanout). Without a
+    backward there is nothing to join, and autocast may hold a weight's cast
+    from one call for the next, which a decoding loop's few rows live from,
+    also where gradients are on."""
     ws = [getattr(m, "weight", None) for m in mods]
     if (x.dtype == torch.bfloat16 and x.is_cuda and torch.is_grad_enabled()
             and x.numel() >= 64 * x.shape[-1] > 0
@@ -350,6 +351,7 @@ def linears(x, mods):
             and all(_plain_linear(m) for m in mods) and not _global_hooks()
             and all(w.dtype == ws[0].dtype and w.device == x.device and w.is_contiguous()
                     and w.shape[1] == x.shape[-1] for w in ws)
+            and (x.requires_grad or any(w.requires_grad for w in ws))
             and ws[0].dtype in _PACKED[_autocast()] and not torch.compiler.is_compiling()):
         return list(_LinearsFn.apply(x, _PackFn.apply(*ws), [w.shape[0] for w in ws]))
     return [m(xi) for m, xi in zip(mods, fanout(x, len(mods)))]

@@ -6,7 +6,7 @@ import pytest
 import torch
 import torch.nn as nn
 
-from nested_recurrent_memory_amd.layer_ops import _plain_linear, first_linear
+from nested_recurrent_memory_amd.layer_ops import _LinearsFn, _plain_linear, first_linear, linears
 
 
 def _linear():
@@ -38,3 +38,19 @@ def test_a_global_hook_sees_the_sequential(register):
     finally:
         handle.remove()
     assert first_linear(seq) is seq[0]
+
+
+@pytest.mark.gpu
+def test_nothing_to_differentiate_runs_the_modules(monkeypatch):
+    """Gradients on, but neither x nor a weight wants one (an evaluation
+    without no_grad): no weight is cast into a pack that nothing needs."""
+    mods = [nn.Linear(64, n, bias=False).cuda().requires_grad_(False) for n in (64, 32)]
+    x = torch.randn(64, 64, device="cuda").bfloat16()
+    with monkeypatch.context() as mp, torch.autocast("cuda", dtype=torch.bfloat16):
+        mp.setattr(_LinearsFn, "apply", lambda *a: pytest.fail("joined"))
+        assert all(torch.equal(y, m(x)) for y, m in zip(linears(x, mods), mods))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        for leaf in (x, mods[1].weight):
+            leaf.requires_grad_(True)
+            assert type(linears(x, mods)[0].grad_fn).__name__ == "_LinearsFnBackward"
+            leaf.requires_grad_(False)
