@@ -18,6 +18,7 @@ on tensors off the GPU) the calls raise.
 from __future__ import annotations
 
 import ctypes
+import itertools
 
 import torch
 import torch.nn as nn
@@ -259,9 +260,13 @@ class _PackFn(torch.autograd.Function):
         parts = dw.split(ctx.ns)
         if torch.is_grad_enabled():        # a gradient that is differentiated again
             return tuple(p.to(ctx.dtype) for p in parts)
-        out = [torch.empty(p.shape, device=p.device, dtype=ctx.dtype) for p in parts]
-        torch._foreach_copy_(out, list(parts))
-        return tuple(o if need else None for o, need in zip(out, ctx.needs_input_grad))
+        wanted = [i for i, need in enumerate(ctx.needs_input_grad) if need]
+        out = [torch.empty(parts[i].shape, device=dw.device, dtype=ctx.dtype) for i in wanted]
+        torch._foreach_copy_(out, [parts[i] for i in wanted])
+        grads = [None] * len(parts)
+        for i, g in zip(wanted, out):
+            grads[i] = g
+        return tuple(grads)
 
 
 def _cat_columns(xs):
@@ -283,9 +288,10 @@ class _LinearsFn(torch.autograd.Function):
     seven adds and fourteen GEMMs fewer, the host and the card both."""
 
     @staticmethod
-    def forward(ctx, x, w, ns):
+    def forward(ctx, x, w, ns, needs):
+        """needs: whether each map's weight wants its gradient."""
         ctx.save_for_backward(x, w)
-        ctx.ns = ns
+        ctx.ns, ctx.needs = ns, needs
         x2 = x.reshape(-1, x.shape[-1])
         return tuple(torch.mm(x2, p.t()).view(*x.shape[:-1], p.shape[0]) for p in w.split(ns))
 
@@ -301,8 +307,19 @@ class _LinearsFn(torch.autograd.Function):
             if ctx.needs_input_grad[0]:
                 dx = torch.mm(dy, w).view(x.shape)
             if ctx.needs_input_grad[1]:
-                dw = torch.mm(dy.t(), x2)
-        return dx, dw, None
+                if all(ctx.needs) or torch.is_grad_enabled():
+                    dw = torch.mm(dy.t(), x2)
+                else:            # one product per run of wanted weights, zeros between
+                    dw = torch.empty_like(w)
+                    a = 0
+                    for need, run in itertools.groupby(zip(ctx.needs, ctx.ns), lambda t: t[0]):
+                        b = a + sum(n for _, n in run)
+                        if need:
+                            torch.mm(dy[:, a:b].t(), x2, out=dw[a:b])
+                        else:
+                            dw[a:b].zero_()
+                        a = b
+        return dx, dw, None, None
 
 
 def _no_hooks(m):
@@ -353,7 +370,8 @@ def linears(x, mods):
                     and w.shape[1] == x.shape[-1] for w in ws)
             and (x.requires_grad or any(w.requires_grad for w in ws))
             and ws[0].dtype in _PACKED[_autocast()] and not torch.compiler.is_compiling()):
-        return list(_LinearsFn.apply(x, _PackFn.apply(*ws), [w.shape[0] for w in ws]))
+        return list(_LinearsFn.apply(x, _PackFn.apply(*ws), [w.shape[0] for w in ws],
+                                     [w.requires_grad for w in ws]))
     return [m(xi) for m, xi in zip(mods, fanout(x, len(mods)))]
 
 

@@ -6,7 +6,8 @@ import pytest
 import torch
 import torch.nn as nn
 
-from nested_recurrent_memory_amd.layer_ops import _LinearsFn, _plain_linear, first_linear, linears
+from nested_recurrent_memory_amd.layer_ops import (_LinearsFn, _PackFn, _plain_linear,
+                                                   first_linear, linears)
 
 
 def _linear():
@@ -54,3 +55,24 @@ def test_nothing_to_differentiate_runs_the_modules(monkeypatch):
             leaf.requires_grad_(True)
             assert type(linears(x, mods)[0].grad_fn).__name__ == "_LinearsFnBackward"
             leaf.requires_grad_(False)
+
+
+@pytest.mark.parametrize("needs", [(False, True, False, False), (True, False, False, True),
+                                   (True, True, True, True), (False, True, True, False)])
+def test_only_wanted_weight_gradients_are_formed(needs, monkeypatch):
+    """The rows of weights that want no gradient are neither multiplied nor
+    handed on; the others are those of one product."""
+    ns, d, rows = (8, 24, 3, 16), 16, 64
+    gen = torch.Generator().manual_seed(0)
+    ws = [torch.randn(n, d, generator=gen).bfloat16().requires_grad_(r) for n, r in zip(ns, needs)]
+    x = torch.randn(rows, d, generator=gen).bfloat16().requires_grad_(True)
+    dys = [torch.randn(rows, n, generator=gen).bfloat16() for n in ns]
+    ys = _LinearsFn.apply(x, _PackFn.apply(*ws), ns, needs)
+    formed, mm = [], torch.mm
+    monkeypatch.setattr(torch, "mm", lambda a, b, **kw: formed.append(a.shape[0]) or mm(a, b, **kw))
+    torch.autograd.backward(ys, dys)
+    assert sum(formed) == rows + sum(n for n, r in zip(ns, needs) if r)      # dx, and dw
+    for w, dy, r in zip(ws, dys, needs):
+        assert (w.grad is not None) == r
+        # bf16 results of the same fp32 sums, 2^-9 of each value
+        assert not r or (w.grad - dy.t() @ x).float().norm() <= 2 ** -8 * w.grad.float().norm()
