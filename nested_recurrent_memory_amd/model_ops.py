@@ -288,6 +288,9 @@ class _LinearCEFn(torch.autograd.Function):
                     if bc is not None:
                         pb = logits.float().sum(0)
                         db = pb if db is None else db.add_(pb)
+        if grad and N == 0:        # no block ran
+            dx, dw = torch.empty_like(xc), torch.zeros_like(wc)
+            db = torch.zeros_like(bc) if bc is not None else None
         ctx.dtypes = (x.dtype, weight.dtype, bias.dtype if bias is not None else None)
         ctx.card_bound = card_bound
         if grad:

@@ -57,3 +57,20 @@ def test_loss_gradients_in_blocks_and_differentiated_again(wdtype, monkeypatch):
     for a, b in zip(one, grads()):
         # each block's gradient rounded to bf16 (2^-9 of a value) before the fp32 sum
         assert a.dtype == b.dtype and (a - b).float().norm() <= 2 ** -8 * a.float().norm()
+
+
+@pytest.mark.parametrize("wants", [(True, False, False), (True, True, True), (False, True, False)])
+def test_loss_of_no_tokens(wants):
+    """An empty batch: loss 0, and gradients of zeros in the inputs' shapes
+    and types, whichever of them are wanted (a frozen head among them)."""
+    x = torch.randn(0, 24, device="cuda").requires_grad_(wants[0])
+    w = torch.randn(104, 24, device="cuda").requires_grad_(wants[1])
+    b = torch.randn(104, device="cuda").requires_grad_(wants[2])
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        loss = model_ops.fused_linear_cross_entropy(x, torch.zeros(0, device="cuda", dtype=torch.long),
+                                                    w, b)
+    loss.backward()
+    assert loss.item() == 0.0
+    for t, want in zip((x, w, b), wants):
+        assert (t.grad is not None) == want
+        assert not want or (t.grad.shape == t.shape and t.grad.dtype == t.dtype and not t.grad.any())
