@@ -211,7 +211,8 @@ class _Layout:
 
     def add(self, name, *shape, es=4, batched=True):
         n = math.prod(shape) * es
-        self.at[name] = (self.bytes, n // shape[0] if batched else 0, shape)
+        row = n // shape[0] if batched and shape[0] else 0
+        self.at[name] = (self.bytes, row, shape)
         self.bytes += -(-n // 256) * 256
 
     def ptrs(self, base, b0=0):
