@@ -204,15 +204,16 @@ def _run_groups(B, dev, launch):
 
 class _Layout:
     """Buffers in one allocation: name -> (byte offset, bytes per batch row,
-    shape), 256-byte aligned; row 0 for buffers without a batch axis."""
+    shape), 256-byte aligned; row 0 for buffers without a batch axis.
+    ``es``: name -> bytes per value (4: fp32, 2: bf16)."""
 
     def __init__(self):
-        self.at, self.bytes = {}, 0
+        self.at, self.es, self.bytes = {}, {}, 0
 
     def add(self, name, *shape, es=4, batched=True):
         n = math.prod(shape) * es
         row = n // shape[0] if batched and shape[0] else 0
-        self.at[name] = (self.bytes, row, shape)
+        self.at[name], self.es[name] = (self.bytes, row, shape), es
         self.bytes += -(-n // 256) * 256
 
     def ptrs(self, base, b0=0):
@@ -328,8 +329,9 @@ class _Saved(dict):
 
     def buffer(self, name):
         o, _, shape = self["layout"].at[name]
-        flat = self["kept"][o:o + math.prod(shape) * 4].view(torch.float32)
-        return flat.view(shape)
+        es = self["layout"].es[name]
+        flat = self["kept"][o:o + math.prod(shape) * es]
+        return flat.view(torch.float32 if es == 4 else torch.bfloat16).view(shape)
 
     def __missing__(self, name):
         if name in ("states", "statesT"):

@@ -30,3 +30,17 @@ def test_no_rows_is_refused_by_the_library(L):
     args = {n: (x.cuda() if n in LEAVES else x) for n, x in args.items()}
     with pytest.raises(_lib.NgdnError, match="bad sizes B=0"):
         chunk_nested_gdn2(**args, L=L)
+
+
+@pytest.mark.parametrize("es,dtype", [(2, torch.bfloat16), (4, torch.float32)])
+def test_a_kept_buffer_has_its_own_type(es, dtype):
+    """The parameter layouts are of the working type, all else fp32; every
+    view lies inside the kept allocation."""
+    kept, _, levels = _layout(2, es=es)
+    saved = chunk_mod._Saved(kept=torch.zeros(kept.bytes, dtype=torch.uint8), layout=kept,
+                             levels=levels)
+    for name, (_, _, shape) in kept.at.items():
+        params = name in ("bpT", "wpT", "gpT", "kpT", "bankT")
+        assert saved[name].shape == shape
+        assert saved[name].dtype == (dtype if params else torch.float32), name
+    assert saved["bpT"].shape == (2, 2, 64, 64) and saved["states"][0] is None
