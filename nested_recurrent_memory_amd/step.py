@@ -184,6 +184,9 @@ def step_nested_gdn2(
             par = params
             if par["qb"].dtype != wd:
                 raise ValueError(f"params were prepared for {par['qb'].dtype}, inputs are {wd}")
+        elif not all(x.is_cuda for x in (b_projections, w_projections, g_projections)
+                     + (() if merge else (query_banks, key_projections))):
+            raise ValueError("step_nested_gdn2 runs on the GPU only; got parameters off it")
         elif pos_t is None and not any((pos_all + 1) % (int(chunk_size) * x) == 0 for x in f[1:]):
             # a host position at which no level fires: the parameters are not
             # read, and are not laid out either (63 of 64 tokens; one sequence,

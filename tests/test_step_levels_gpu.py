@@ -34,3 +34,15 @@ def test_step_levels(dtype, L, K, inplace):
     o_r, s_r = ref.step_forward(*(tok[n].double() for n in TOKEN), state.double(), pos,
                                 *(x.double() for x in rest[:5]), *rest[5:], L=L)
     _parity.check_all([("o", o, o_r), ("state", s_new, s_r)], dtype, test=f"step_L{L}")
+
+
+@pytest.mark.parametrize("name", ["query_banks", "key_projections", "b_projections", "w_projections",
+                                  "g_projections"])
+@pytest.mark.parametrize("position", [5, 63])      # the level does not fire; it does
+def test_step_refuses_parameters_off_the_gpu(name, position):
+    inp = make_inputs(B=1, T=1, H=2, K=64, V=64, L=2, N=16, intervals=(1, 1), dtype=torch.bfloat16)
+    args = {n: (inp[n][:, 0] if n in TOKEN else inp[n]) for n in NAMES}
+    args = {n: x if n == name else x.cuda() for n, x in args.items()}
+    with torch.no_grad(), pytest.raises(ValueError, match="GPU"):
+        step_nested_gdn2(**args, state=torch.zeros(1, 2, 2, 64, 64, device="cuda"), position=position,
+                         L=2)
