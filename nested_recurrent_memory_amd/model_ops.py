@@ -222,7 +222,9 @@ _BLOCK_BYTES = 4 << 30     # logits held at once
 # not the host sets its time: three products of 2^35 at 1.0 PFLOP/s take 0.2
 # ms, the host's calls 0.24 ms. Below, ngdn_scale's own call costs more host
 # time than torch's (128 x 512 x 8000: 255 against 232 us a pass); above, it
-# saves passes (8192 x 1024 x 32000: 1619 against 1695).
+# saves passes (8192 x 1024 x 32000: 1619 against 1695). Below, the gradient of
+# an fp32 x is also rounded to bf16 after the factor, which torch's product is
+# formed in; above, only before it.
 _CARD_BOUND = 1 << 35
 _SCALED = (torch.float32, torch.bfloat16)
 
